@@ -4,7 +4,9 @@ test_gpu_parity: particles in slot order, counters, sampler and wall sums)."""
 import pytest
 
 from test_gpu_parity import assert_identical, pair
-from unigasfoam_amd import workloads
+from unigasfoam_amd import abi, workloads
+from unigasfoam_amd.mesh import box_mesh
+from unigasfoam_amd.spec import Boundary, CaseSpec
 
 pytestmark = pytest.mark.gpu
 
@@ -19,3 +21,26 @@ def test_many_cells_crossed_per_step_identical(require_gpu, n, per_cell, stretch
     g.step(6)
     o.step(6)
     assert_identical(g, o, f"{n}^3 cells, {per_cell} each")
+
+
+@pytest.mark.parametrize("cells,per_cell", [((1, 1, 1), 7), ((1, 1, 1), 700), ((5, 3, 2), 150), ((65, 64, 1), 3),
+                                            ((65, 64, 1), 90)])
+@pytest.mark.parametrize("kind", [abi.BND_SPECULAR, abi.BND_DIFFUSE])
+def test_wall_sums_of_few_and_many_hits_identical(require_gpu, cells, per_cell, kind):
+    """Two species between measured walls in a flat box: faces with no hit, a
+    few, and more than the sort stages at a time, with a wave per face (up to
+    8192 faces) and with sixteen lanes (65 x 64 x 1 has 8578)."""
+    pt = {k: abi.WALL for k in ("xmin", "xmax", "ymin", "ymax", "zmin", "zmax")}
+    size = (1.0e-3 * cells[0], 1.0e-3 * cells[1], 2.0e-4 * cells[2])
+    mesh = box_mesh((0.0, 0.0, 0.0), size, cells, pt)
+    n = 1.0e20
+    spec = CaseSpec(mesh=mesh, species=[workloads.N2, workloads.ARGON], delta_t=4.0e-7,
+                    n_equivalent_particles=n * size[0] * size[1] * size[2] / (per_cell * mesh.n_cells),
+                    collision_model="dsmc", dsmc_model="LarsenBorgnakkeVariableHardSphere", Tref=273.0, seed=9,
+                    boundaries=[Boundary(p, kind, 400.0, (30.0, 0.0, 0.0)) for p in sorted(pt)])
+    g, o = pair(spec, dict(number_density={"N2": 0.6 * n, "Ar": 0.4 * n}, T=300.0),
+                capacity=1 << 22)   # the event buffers hold an eighth of it
+    g.step(2)
+    o.step(2)
+    assert g.counters()["wall_hits"] > 0
+    assert_identical(g, o, f"{cells} cells, {per_cell} each")

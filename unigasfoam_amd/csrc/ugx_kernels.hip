@@ -960,105 +960,154 @@ __global__ void k_clone_finish(WorldView<R> w)
 // (uniGasPatchBoundary.C:130-302 measures in the order of the cloud's list).
 
 template <class R>
-__global__ void k_wall_count(WorldView<R> w)
-{
-    const uint32_t n = min(w.st->nev, w.ev_cap);
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
-        atomicAdd(&w.wcnt[w.ev[i].wf], 1u);
-}
-
-template <class R>
 __global__ void k_wall_bucket(WorldView<R> w)
 {
-    const uint32_t n = min(w.st->nev, w.ev_cap);
+    const uint32_t n = w.st->nev;
+    if (n > w.ev_cap) return;   // the step is in error (evover)
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-        const uint32_t wf = w.ev[i].wf;
-        const uint32_t pos = w.woff[wf] + atomicAdd(&w.wcnt[wf], 1u);
+        const uint32_t pos = w.woff[w.ev[i].wf] + w.ev[i].rank;
         w.bkey[pos] = w.ev_key[i];
         w.bidx[pos] = i;
     }
 }
 
-// In-place heap sort of n keys (ascending), carrying their values.
-__device__ inline void heap_sort(unsigned long long* k, uint32_t* v, uint32_t n)
-{
-    auto sift = [&](uint32_t root, uint32_t end) {
-        for (;;) {
-            uint32_t ch = 2u * root + 1u;
-            if (ch >= end) break;
-            if (ch + 1u < end && k[ch] < k[ch + 1u]) ch += 1u;
-            if (!(k[root] < k[ch])) break;
-            const unsigned long long tk = k[root]; k[root] = k[ch]; k[ch] = tk;
-            const uint32_t tv = v[root]; v[root] = v[ch]; v[ch] = tv;
-            root = ch;
-        }
-    };
-    for (uint32_t s = n / 2u; s-- > 0u;) sift(s, n);
-    for (uint32_t e = n; e-- > 1u;) {
-        const unsigned long long tk = k[0]; k[0] = k[e]; k[e] = tk;
-        const uint32_t tv = v[0]; v[0] = v[e]; v[e] = tv;
-        sift(0u, e);
-    }
-}
-
 // measurePropertiesBeforeControl / AfterControl terms of one velocity and
-// E_rot (uniGasPatchBoundary.C:147-184, 223-254) added to a[0..9].
+// E_rot (uniGasPatchBoundary.C:147-184, 223-254): t[0..9].
 __device__ inline void wall_terms(const double U[3], double e, const double n[3], double fA, double m, int rotdof,
-                                  double a[kWRows])
+                                  double t[UGX_W_ROTDOF + 1])
 {
     const double Un = U[0] * n[0] + U[1] * n[1] + U[2] * n[2];
     const double inv = 1.0 / fmax(fabs(Un) * fA, kVSmall);
     const double UU = U[0] * U[0] + U[1] * U[1] + U[2] * U[2];
-    a[UGX_W_RHON] += inv;
-    if (rotdof > 0) a[UGX_W_RHON_INT] += inv;
-    a[UGX_W_RHOM] += m * inv;
-    a[UGX_W_LINEAR_KE] += 0.5 * m * UU * inv;
-    a[UGX_W_MCC] += m * UU * inv;
-    a[UGX_W_MU] += m * U[0] * inv;
-    a[UGX_W_MV] += m * U[1] * inv;
-    a[UGX_W_MW] += m * U[2] * inv;
-    a[UGX_W_EROT] += e * inv;
-    a[UGX_W_ROTDOF] += (double)rotdof * inv;
+    t[UGX_W_RHON] = inv;
+    t[UGX_W_RHON_INT] = (rotdof > 0) ? inv : 0.0;
+    t[UGX_W_RHOM] = m * inv;
+    t[UGX_W_LINEAR_KE] = 0.5 * m * UU * inv;
+    t[UGX_W_MCC] = m * UU * inv;
+    t[UGX_W_MU] = m * U[0] * inv;
+    t[UGX_W_MV] = m * U[1] * inv;
+    t[UGX_W_MW] = m * U[2] * inv;
+    t[UGX_W_EROT] = e * inv;
+    t[UGX_W_ROTDOF] = (double)rotdof * inv;
 }
 
-// One thread per wall face: sort its bucket, sum each species' hits in key
-// order, and add deltaT times the sums at sample steps.
-template <class R>
+// A group of G lanes per wall face: sorts the face's hits by key and adds
+// each species' terms in that order, then deltaT times the sums to the face's
+// time sums (at sample steps).  The order of the additions is fixed, so what
+// runs in parallel is the sort (each hit's place is the number of smaller
+// keys; keys are distinct) and the terms of a chunk of hits, which go to LDS;
+// then lane r adds row r of the chunk, hit after hit.  One thread per face
+// with a heap sort in HBM took 149 us per step for the two faces of a 1-D
+// channel (60 hits each) and 65 us for a box of 3174 faces (8 hits each): a
+// serial chain of dependent memory reads.  Here: 17 and 9 us.
+template <class R, int G>
 __global__ void __launch_bounds__(kBlock) k_wall_reduce(WorldView<R> w)
 {
-    const uint32_t f = blockIdx.x * blockDim.x + threadIdx.x;
-    if (f >= (uint32_t)w.nwf) return;
-    const uint32_t b = w.woff[f], e = w.woff[f + 1];
-    if (e == b) return;
+    constexpr uint32_t kGroups = kBlock / G;
+    constexpr uint32_t kKeys = 4u * G;             // keys staged at a time
+    constexpr uint32_t kChunk = (G == 64) ? 32u : 8u;   // hits whose terms are staged at a time
+    constexpr int kPair = UGX_W_ROTDOF + 1;        // rows with a term before and one after the wall
+    constexpr int kTerms = 2 * kPair + (kWRows - kPair);
+    static_assert(kWRows <= G && kChunk <= (uint32_t)G, "a lane per row and per staged hit");
+    __shared__ unsigned long long s_key[kGroups][kKeys];
+    __shared__ uint32_t s_ord[kGroups][kKeys];
+    __shared__ double s_t[kGroups][kTerms][kChunk + 1];
+    __shared__ uint32_t s_sp[kGroups][kChunk];
+    const uint32_t gi = threadIdx.x / G, j = threadIdx.x % G;
+    const uint32_t f = blockIdx.x * kGroups + gi;
+    if (f >= (uint32_t)w.nwf || w.st->nev > w.ev_cap) return;
+    const uint32_t b = w.woff[f], n = w.woff[f + 1] - b;
+    if (n == 0u) return;
     const CaseDev& cs = w.cases[w.cell_case[w.wcell[f]]];
     if (((cs.step + 1u) % (uint32_t)cs.sample_interval) != 0u) return;
-    heap_sort(w.bkey + b, w.bidx + b, e - b);
+    // the order: in LDS, or for a face with more hits in the key list, whose
+    // contents the buckets hold (entries b.. of it are this face's to use)
+    const bool small = n <= kKeys;
+    uint32_t* const ord = reinterpret_cast<uint32_t*>(w.ev_key) + b;
+    for (uint32_t q0 = 0; q0 < n; q0 += kKeys) {
+        unsigned long long mk[4];
+        uint32_t mr[4] = {0u, 0u, 0u, 0u};
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const uint32_t q = q0 + j + G * (uint32_t)u;
+            mk[u] = (q < n) ? w.bkey[b + q] : 0ull;
+        }
+        for (uint32_t p0 = 0; p0 < n; p0 += kKeys) {
+            wave_sync();
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const uint32_t p = p0 + j + G * (uint32_t)u;
+                if (p < n) s_key[gi][j + G * (uint32_t)u] = w.bkey[b + p];
+            }
+            wave_sync();
+            const uint32_t pn = min(kKeys, n - p0);
+            for (uint32_t p = 0; p < pn; ++p) {
+                const unsigned long long k = s_key[gi][p];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) mr[u] += (k < mk[u]) ? 1u : 0u;
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const uint32_t q = q0 + j + G * (uint32_t)u;
+            if (q >= n) continue;
+            if (small) s_ord[gi][mr[u]] = w.bidx[b + q];
+            else ord[mr[u]] = w.bidx[b + q];
+        }
+    }
+    if (!small) __threadfence_block();
+    wave_sync();
     const double* gq = &w.wgeo[(size_t)f * kWGeo];
-    const double n[3] = {gq[0], gq[1], gq[2]};
+    const double nw[3] = {gq[0], gq[1], gq[2]};
     const double fA = gq[3];
     // nParticle F_N W_c of the face's cell (uniGasPatchBoundary.C:292-294)
     const double FN = cs.fn * w.cw[w.wcell[f]], dt = cs.dt;
-    uint32_t i = b;
-    while (i < e) {
-        const uint32_t ls = (uint32_t)(w.bkey[i] >> 42);
-        const uint32_t g = (uint32_t)cs.sp_base + ls;
-        const double m = w.sp.mass[g];
-        const int rotdof = w.sp.rotdof[g];
-        double a[kWRows];
-        for (int r = 0; r < kWRows; ++r) a[r] = 0.0;
-        for (; i < e && (uint32_t)(w.bkey[i] >> 42) == ls; ++i) {
-            const WallEv ev = w.ev[w.bidx[i]];
-            wall_terms(ev.u0, ev.e0, n, fA, m, rotdof, a);
+    double* const sums = &w.wsamp[(size_t)f * kNS * kWRows];
+    double a = 0.0;
+    int ls = -1;
+    for (uint32_t p0 = 0; p0 < n; p0 += kChunk) {
+        const uint32_t pn = min(kChunk, n - p0);
+        if (j < pn) {
+            const WallEv ev = w.ev[small ? s_ord[gi][p0 + j] : ord[p0 + j]];
+            const double m = w.sp.mass[ev.sp];
+            const int rotdof = w.sp.rotdof[ev.sp];
+            double t0[kPair], t1[kPair];
+            wall_terms(ev.u0, ev.e0, nw, fA, m, rotdof, t0);
             const double preIE = 0.5 * m * (ev.u0[0] * ev.u0[0] + ev.u0[1] * ev.u0[1] + ev.u0[2] * ev.u0[2]) + ev.e0;
-            wall_terms(ev.u1, ev.e1, n, fA, m, rotdof, a);
+            wall_terms(ev.u1, ev.e1, nw, fA, m, rotdof, t1);
             const double postIE = 0.5 * m * (ev.u1[0] * ev.u1[0] + ev.u1[1] * ev.u1[1] + ev.u1[2] * ev.u1[2]) + ev.e1;
-            a[UGX_W_Q] += FN * (preIE - postIE) / (dt * fA);
-            for (int d = 0; d < 3; ++d) a[UGX_W_FX + d] += FN * (m * ev.u0[d] - m * ev.u1[d]) / (dt * fA);
+#pragma unroll
+            for (int r = 0; r < kPair; ++r) { s_t[gi][r][j] = t0[r]; s_t[gi][kPair + r][j] = t1[r]; }
+            s_t[gi][2 * kPair][j] = FN * (preIE - postIE) / (dt * fA);
+            for (int d = 0; d < 3; ++d)
+                s_t[gi][2 * kPair + 1 + d][j] = FN * (m * ev.u0[d] - m * ev.u1[d]) / (dt * fA);
+            s_sp[gi][j] = ev.sp - (uint32_t)cs.sp_base;
         }
-        double* dst = &w.wsamp[((size_t)f * kNS + ls) * kWRows];
-        for (int r = 0; r < kWRows; ++r) dst[r] += dt * a[r];
+        wave_sync();
+        if (j < (uint32_t)kWRows) {
+            const bool pair = j < (uint32_t)kPair;
+            const double* ta = s_t[gi][pair ? j : j + kPair];
+            const double* tb = s_t[gi][pair ? j + kPair : j + kPair];
+            for (uint32_t i = 0; i < pn; ++i) {
+                const int s = (int)s_sp[gi][i];
+                if (s != ls) {
+                    if (ls >= 0) sums[(size_t)ls * kWRows + j] += dt * a;
+                    a = 0.0;
+                    ls = s;
+                }
+                a += ta[i];
+                if (pair) a += tb[i];
+            }
+        }
+        wave_sync();
     }
+    if (j < (uint32_t)kWRows && ls >= 0) sums[(size_t)ls * kWRows + j] += dt * a;
 }
+
+// Up to this many wall faces a wave each: the waves are then resident at once
+// (256 CUs x 32).  More faces (a 3-D mesh, few hits each) take 16 lanes each:
+// 45,000 faces with one hit each take 21 us (23 us with a thread per face).
+constexpr int32_t kWallWaveFaces = 8192;
 
 // ------------------------------------------------------------ occupancy
 // The sort after the move needs each cell's new population and, for every
@@ -3665,6 +3714,8 @@ void launch_step(const WorldView<R>& w0, hipStream_t s, hipEvent_t* marks)
     hipLaunchKernelGGL(k_begin_step<R>, dim3(gc), dim3(kBlock), 0, s, w);
     hipLaunchKernelGGL(k_zero_u32, dim3(grid_for(ncp)), dim3(kBlock), 0, s, w.cnt, ncp);
     hipLaunchKernelGGL(k_zero_u32, dim3(grid_for(ncp)), dim3(kBlock), 0, s, w.ocnt, ncp);
+    if (w.nwf > 0)
+        hipLaunchKernelGGL(k_zero_u32, dim3(grid_for((uint64_t)w.nwf + 1)), dim3(kBlock), 0, s, w.wcnt, (uint32_t)w.nwf + 1u);
     mark(1);
     if (w.n_inflow > 0) {
         if (w.n_inflow > 4096) {
@@ -3683,12 +3734,13 @@ void launch_step(const WorldView<R>& w0, hipStream_t s, hipEvent_t* marks)
     hipLaunchKernelGGL(k_wall<R>, dim3(grid_for(w.wq_cap, 2048)), dim3(kBlock), 0, s, w);
     if (w.nwf > 0) {
         const uint32_t nw1 = (uint32_t)w.nwf + 1u;
-        hipLaunchKernelGGL(k_zero_u32, dim3(grid_for(nw1)), dim3(kBlock), 0, s, w.wcnt, nw1);
-        hipLaunchKernelGGL(k_wall_count<R>, dim3(grid_for(w.ev_cap, 1024)), dim3(kBlock), 0, s, w);
         scan_u32(w.wcnt, nw1, w.woff, w.blocksum, nullptr, s);
-        hipLaunchKernelGGL(k_zero_u32, dim3(grid_for(nw1)), dim3(kBlock), 0, s, w.wcnt, nw1);
         hipLaunchKernelGGL(k_wall_bucket<R>, dim3(grid_for(w.ev_cap, 1024)), dim3(kBlock), 0, s, w);
-        hipLaunchKernelGGL(k_wall_reduce<R>, dim3(grid_for((uint64_t)w.nwf)), dim3(kBlock), 0, s, w);
+        if (w.nwf <= kWallWaveFaces)
+            hipLaunchKernelGGL((k_wall_reduce<R, 64>), dim3(grid_for((uint64_t)w.nwf * 64)), dim3(kBlock), 0, s, w);
+        else
+            hipLaunchKernelGGL((k_wall_reduce<R, 16>), dim3((unsigned)(((uint64_t)w.nwf * 16 + kBlock - 1) / kBlock)),
+                               dim3(kBlock), 0, s, w);
     }
     if (w.has_weighting) {
         const unsigned gw = count_grid(w.cap);

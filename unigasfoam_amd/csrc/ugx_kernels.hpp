@@ -29,6 +29,8 @@ struct WallEv {
     double e0, e1;
     uint32_t wf;
     uint32_t sp;
+    uint32_t rank;          // arrival number among the step's hits of the face
+    uint32_t pad;
 };
 // Rows of the wall sums per (face, species): ugx_wall_index.
 constexpr int kWRows = UGX_W_COUNT;
@@ -203,6 +205,7 @@ struct WallSink {
     const int32_t* wface;
     WallEv* ev;
     unsigned long long* key;
+    uint32_t* cnt;            // hits per wall face, zero at the start of a step
     uint32_t cap;
     DevState* st;
     const int32_t* local;
@@ -218,7 +221,10 @@ struct WallSink {
                         double e1, uint32_t sp) const
     {
         const int32_t wf = wface[(size_t)c * kMaxFaces + f];
+        // both numbers in one round trip; past the capacity the step is reported
+        // as an error and its hits are not reduced
         const uint32_t i = atomicAdd(&st->nev, 1u);
+        const uint32_t rank = atomicAdd(&cnt[wf], 1u);
         if (i >= cap) { st->evover = 1u; return; }
         key[i] = ((unsigned long long)(uint32_t)local[sp] << 42) | ((unsigned long long)slot << 10) |
                  (unsigned long long)(uint32_t)ord;
@@ -228,6 +234,8 @@ struct WallSink {
         e.e1 = e1;
         e.wf = (uint32_t)wf;
         e.sp = sp;
+        e.rank = rank;
+        e.pad = 0u;
         ev[i] = e;
     }
 };
@@ -235,7 +243,7 @@ struct WallSink {
 template <class R>
 __device__ inline WallSink wall_sink(const WorldView<R>& w)
 {
-    return WallSink{w.nwf > 0 ? w.wface : nullptr, w.ev, w.ev_key, w.ev_cap, w.st, w.sp.local, w.cell_case, w.cases};
+    return WallSink{w.nwf > 0 ? w.wface : nullptr, w.ev, w.ev_key, w.wcnt, w.ev_cap, w.st, w.sp.local, w.cell_case, w.cases};
 }
 
 // Rows of the per-cell sums kept for the BGK family: every base row and the
