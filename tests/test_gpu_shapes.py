@@ -1,10 +1,12 @@
 """The step's kernels at the sizes where their work division changes: GPU
 (FP64) against the CPU oracle, bit for bit (assert_identical of
 test_gpu_parity: particles in slot order, counters, sampler and wall sums)."""
+import numpy as np
 import pytest
 
 from test_gpu_parity import assert_identical, pair
 from unigasfoam_amd import abi, workloads
+from unigasfoam_amd.core import Case
 from unigasfoam_amd.mesh import box_mesh
 from unigasfoam_amd.spec import Boundary, CaseSpec
 
@@ -44,3 +46,30 @@ def test_wall_sums_of_few_and_many_hits_identical(require_gpu, cells, per_cell, 
     o.step(2)
     assert g.counters()["wall_hits"] > 0
     assert_identical(g, o, f"{cells} cells, {per_cell} each")
+
+
+@pytest.mark.parametrize("n", [1, 255, 256, 1023, 1024, 1025, 2048])
+def test_offsets_at_block_edges_identical(require_gpu, n):
+    """Cell counts around the blocks of the offset scan (1024 cells each)."""
+    spec, fill = workloads.couette(n_cells=n, per_cell=5)
+    g, o = pair(spec, fill)
+    g.step(5)
+    o.step(5)
+    assert_identical(g, o, f"{n} cells")
+
+
+def test_offsets_of_more_than_4096_blocks(require_gpu):
+    """4.3e6 cells: the scan's block sums are scanned first.  Every simulator
+    is where the sampler counted it, in cell order, and none is lost."""
+    spec, fill = workloads.heat_bath(n_cells=162, per_cell=1, side=0.162)
+    g = Case(spec, precision="fp32")
+    g.fill(**fill)
+    g.step(2)
+    cell = g.particles()["cell"]
+    assert cell.size == 162 ** 3
+    assert np.all(np.diff(cell) >= 0)
+    g.reset_samples()
+    g.step(1)
+    cell = g.particles()["cell"]
+    assert np.all(np.diff(cell) >= 0)
+    assert np.array_equal(g.samples()[abi.S["N"]] / spec.delta_t, np.bincount(cell, minlength=162 ** 3))

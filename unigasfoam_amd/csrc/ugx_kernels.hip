@@ -186,64 +186,95 @@ __device__ inline void tcount_block_flush(const TCount<T, M>& t, unsigned long l
     }
 }
 
+__device__ inline uint32_t wave_incl_scan_u32(uint32_t v)
+{
+    const int lane = (int)__lane_id();
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t u = __shfl_up(v, o);
+        if (lane >= o) v += u;
+    }
+    return v;
+}
+
 __global__ void k_zero_u32(uint32_t* p, uint32_t n)
 {
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) p[i] = 0u;
 }
 
+// ------------------------------------------------------------- inflow
+
+// Insert count of face-species k (uniGasGeneralBoundary.C:602-609).
 template <class R>
-__global__ void k_begin_step(WorldView<R> w)
+__device__ inline uint32_t inflow_face(const WorldView<R>& w, int k)
 {
-    int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c < w.ncases) w.cases[c].particle_begin = w.off[w.cases[c].cell_begin];
-    if (c == 0) {
+    const InflowFS& e = w.inflow[k];
+    const CaseDev& cs = w.cases[e.ccase];
+    if (!cs.active) return 0u;
+    Rng r;
+    rng_init(r, cs.seed_lo, cs.seed_hi, kRngInflowN, 0u, (uint32_t)e.local_id, cs.step);
+    // divided by F_N W_c of the face's cell (W_c = 1 unweighted: the same as nbar)
+    const double nb = e.nbar_num / (e.nbar_den * w.cw[e.cell]);
+    const double fl = floor(nb);
+    long long c = (long long)fl;
+    if (c < 0) c = 0;
+    if (uniform(r) < nb - fl) c += 1;
+    return (uint32_t)c;
+}
+
+// The step's inflow total, or none when it would exceed the capacity (the
+// overflow is reported).
+template <class R>
+__device__ inline void inflow_total(const WorldView<R>& w, uint32_t n)
+{
+    if ((unsigned long long)w.st->n + n > (unsigned long long)w.cap) {
+        w.st->overflow = 1u;
+        n = 0u;
+    }
+    w.st->n_ins = n;
+}
+
+// Largest number of face-species counted and scanned by the first block of
+// k_begin_step; more take a thread each and a scan.
+constexpr int kInflowBlock = 4096;
+constexpr int kBeginBlock = 1024;
+
+// Start of a step.  The first block sets the cases' slot bases, the hybrid
+// averaging times and the step's numbers, and counts the inflow of up to
+// kInflowBlock face-species (counts and their exclusive scan); all blocks
+// clear the occupancy counters and the wall-hit counts.  One launch: every
+// launch of a step costs a small run about 4.5 us whatever it does.
+template <class R>
+__global__ void __launch_bounds__(kBeginBlock) k_begin_step(WorldView<R> w)
+{
+    const uint32_t tid = threadIdx.x, gid = blockIdx.x * blockDim.x + tid, gn = gridDim.x * blockDim.x;
+    for (uint32_t i = gid; i <= (uint32_t)w.nc; i += gn) w.ocnt[i] = 0u;
+    if (w.nwf > 0)
+        for (uint32_t i = gid; i <= (uint32_t)w.nwf; i += gn) w.wcnt[i] = 0u;
+    if (blockIdx.x != 0u) return;
+    for (int c = (int)tid; c < w.ncases; c += kBeginBlock) {
+        CaseDev& cs = w.cases[c];
+        cs.particle_begin = w.off[cs.cell_begin];
+        if (cs.active && cs.coll_model == UGX_COLL_HYBRID) cs.kn_time += cs.dt;
+    }
+    if (tid == 0u) {
         w.st->n_ins = 0u; w.st->nwall = 0u; w.st->nsel = 0u;
         w.st->nev_peak = max(w.st->nev_peak, w.st->nev);
         w.st->nev = 0u;
     }
-}
-
-// ------------------------------------------------------------- inflow
-
-// One block: insert counts per face-species (uniGasGeneralBoundary.C:602-609)
-// and their exclusive scan.
-template <class R>
-__global__ void __launch_bounds__(1024) k_inflow_count(WorldView<R> w)
-{
-    __shared__ uint32_t sh[16];
-    const int tid = threadIdx.x;
-    uint32_t carry = 0;
-    for (int base = 0; base < w.n_inflow; base += 1024) {
-        int k = base + tid;
-        uint32_t cnt = 0;
-        if (k < w.n_inflow) {
-            const InflowFS& e = w.inflow[k];
-            const CaseDev& cs = w.cases[e.ccase];
-            if (cs.active) {
-                Rng r;
-                rng_init(r, cs.seed_lo, cs.seed_hi, kRngInflowN, 0u, (uint32_t)e.local_id, cs.step);
-                // divided by F_N W_c of the face's cell (W_c = 1 unweighted: the same as nbar)
-                double nb = e.nbar_num / (e.nbar_den * w.cw[e.cell]);
-                double fl = floor(nb);
-                long long c = (long long)fl;
-                if (c < 0) c = 0;
-                if (uniform(r) < nb - fl) c += 1;
-                cnt = (uint32_t)c;
-            }
-        }
-        // block scan: shuffles within each wave, then the 16 wave totals
-        uint32_t inc = cnt;
-        const int lane = tid & 63;
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const uint32_t u = __shfl_up(inc, o);
-            if (lane >= o) inc += u;
-        }
-        if (lane == 63) sh[tid >> 6] = inc;
+    if (w.n_inflow <= 0 || w.n_inflow > kInflowBlock) return;
+    __shared__ uint32_t sh[kBeginBlock / 64];
+    uint32_t carry = 0u;
+    for (int base = 0; base < w.n_inflow; base += kBeginBlock) {
+        const int k = base + (int)tid;
+        const uint32_t cnt = (k < w.n_inflow) ? inflow_face(w, k) : 0u;
+        // block scan: shuffles within each wave, then the wave totals
+        const uint32_t inc = wave_incl_scan_u32(cnt);
+        if ((tid & 63u) == 63u) sh[tid >> 6] = inc;
         __syncthreads();
         uint32_t below = 0u, tot = 0u;
 #pragma unroll
-        for (int q = 0; q < 16; ++q) {
+        for (uint32_t q = 0; q < kBeginBlock / 64; ++q) {
             const uint32_t v = sh[q];
             if (q < (tid >> 6)) below += v;
             tot += v;
@@ -252,13 +283,9 @@ __global__ void __launch_bounds__(1024) k_inflow_count(WorldView<R> w)
         __syncthreads();
         carry += tot;
     }
-    if (tid == 0) {
+    if (tid == 0u) {
         w.ins_off[w.n_inflow] = carry;
-        if ((unsigned long long)w.st->n + carry > (unsigned long long)w.cap) {
-            w.st->overflow = 1u;
-            carry = 0u;
-        }
-        w.st->n_ins = carry;
+        inflow_total(w, carry);
     }
 }
 
@@ -267,37 +294,15 @@ __global__ void __launch_bounds__(1024) k_inflow_count(WorldView<R> w)
 template <class R>
 __global__ void k_inflow_face_count(WorldView<R> w)
 {
-    for (int k = blockIdx.x * blockDim.x + threadIdx.x; k <= w.n_inflow; k += gridDim.x * blockDim.x) {
-    uint32_t cnt = 0;
-    if (k < w.n_inflow) {
-        const InflowFS& e = w.inflow[k];
-        const CaseDev& cs = w.cases[e.ccase];
-        if (cs.active) {
-            Rng r;
-            rng_init(r, cs.seed_lo, cs.seed_hi, kRngInflowN, 0u, (uint32_t)e.local_id, cs.step);
-            const double nb = e.nbar_num / (e.nbar_den * w.cw[e.cell]);
-            const double fl = floor(nb);
-            long long c = (long long)fl;
-            if (c < 0) c = 0;
-            if (uniform(r) < nb - fl) c += 1;
-            cnt = (uint32_t)c;
-        }
-    }
-    w.ins_off[k] = cnt;
-    }
+    for (int k = blockIdx.x * blockDim.x + threadIdx.x; k <= w.n_inflow; k += gridDim.x * blockDim.x)
+        w.ins_off[k] = (k < w.n_inflow) ? inflow_face(w, k) : 0u;
 }
 
-// After the scan: the step's inflow total, or none when it would exceed the
-// capacity (the overflow is reported).
+// After that scan.
 template <class R>
 __global__ void k_inflow_finish(WorldView<R> w)
 {
-    uint32_t carry = w.ins_off[w.n_inflow];
-    if ((unsigned long long)w.st->n + carry > (unsigned long long)w.cap) {
-        w.st->overflow = 1u;
-        carry = 0u;
-    }
-    w.st->n_ins = carry;
+    inflow_total(w, w.ins_off[w.n_inflow]);
 }
 
 // Bird eq. 12.5 insertion + first move over (1 - R) deltaT.
@@ -349,14 +354,15 @@ __device__ inline int make_inflow(const WorldView<R>& w, const InflowFS& e, cons
     return to.alive;
 }
 
+// The inflow as block `block` of `nblocks`.
 template <class R>
-__global__ void __launch_bounds__(kBlock) k_inflow_gen(WorldView<R> w)
+__device__ inline void inflow_body(const WorldView<R>& w, uint32_t block, uint32_t nblocks,
+                                   TCount<unsigned long long>& tc)
 {
-    TCount<unsigned long long> tc{-1, {0ull, 0ull, 0ull, 0ull}};
     const uint32_t total = w.st->n_ins;
     const uint32_t n0 = w.st->n;
-    const uint32_t stride = gridDim.x * blockDim.x;
-    for (uint32_t base = blockIdx.x * blockDim.x; base < total; base += stride) {
+    const uint32_t stride = nblocks * kBlock;
+    for (uint32_t base = block * kBlock; base < total; base += stride) {
         uint32_t t = base + threadIdx.x;
         bool active = t < total;
         uint32_t cell = kDead;
@@ -393,7 +399,6 @@ __global__ void __launch_bounds__(kBlock) k_inflow_gen(WorldView<R> w)
             tcount_add(tc, w.counters, ccase, 2, (uint32_t)to.errs);
         }
     }
-    tcount_block_flush(tc, w.counters);
 }
 
 // --------------------------------------------------------------- move
@@ -772,15 +777,14 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k
     tcount_block_flush(tc, w.counters);
 }
 
-// Diffuse-wall continuation of the queued tracks.
+// Diffuse-wall continuation of the queued tracks, as block `block` of `nblocks`.
 template <class R>
-__global__ void __launch_bounds__(kBlock) k_wall(WorldView<R> w)
+__device__ inline void wall_body(const WorldView<R>& w, uint32_t block, uint32_t nblocks,
+                                 TCount<unsigned long long>& tc)
 {
-    TCount<unsigned long long> tc{-1, {0ull, 0ull, 0ull, 0ull}};
     const uint32_t nq = min(w.st->nwall, w.wq_cap);
-    const uint32_t stride = gridDim.x * blockDim.x;
-    if (blockIdx.x * blockDim.x >= nq) return;   // nothing to continue, nothing to count
-    for (uint32_t base = blockIdx.x * blockDim.x; base < nq; base += stride) {
+    const uint32_t stride = nblocks * kBlock;
+    for (uint32_t base = block * kBlock; base < nq; base += stride) {
         uint32_t q = base + threadIdx.x;
         bool active = q < nq;
         uint32_t cell = kDead;
@@ -810,6 +814,21 @@ __global__ void __launch_bounds__(kBlock) k_wall(WorldView<R> w)
             tcount_add(tc, w.counters, ccase, 2, (uint32_t)to.errs);
         }
     }
+}
+
+// The continued tracks (the first nwb blocks) and the new simulators (the
+// rest): both are few, long serial chains of FP64 arithmetic and memory round
+// trips that leave the chip mostly idle, and neither needs the other, so they
+// run at the same time (the DSMC nozzle: 16 and 23 us one after the other).
+template <class R>
+__global__ void __launch_bounds__(kBlock) k_wall(WorldView<R> w, uint32_t nwb)
+{
+    const bool walls = blockIdx.x < nwb;
+    const uint32_t block = walls ? blockIdx.x : blockIdx.x - nwb;
+    if (block * kBlock >= (walls ? w.st->nwall : w.st->n_ins)) return;   // nothing to do, nothing to count
+    TCount<unsigned long long> tc{-1, {0ull, 0ull, 0ull, 0ull}};
+    if (walls) wall_body(w, block, nwb, tc);
+    else inflow_body(w, block, gridDim.x - nwb, tc);
     tcount_block_flush(tc, w.counters);
 }
 
@@ -1131,16 +1150,16 @@ constexpr int kCountTiles = 4;                           // tiles per block of k
 // Largest grid of the occupancy count (blocks stride over the step's tile groups).
 constexpr uint64_t kCountGrid = 8192;
 
-// Class-7 counting of the slots [begin, n + n_ins): the inflow of a step, or
-// every slot for the sort after an upload.
+// Class-7 counting of the slots [begin, n + n_ins) as block `block` of
+// `nblocks`: the inflow and clones of a step, or every slot for the sort
+// after an upload.
 template <class R>
-__global__ void k_count(WorldView<R> w, int all)
+__device__ inline void count_slots(const WorldView<R>& w, uint64_t begin, uint32_t block, uint32_t nblocks)
 {
     constexpr int U = kCountUnroll;
     const uint32_t n_all = w.st->n + w.st->n_ins;
-    const uint64_t begin = all ? 0u : w.st->n;
-    const uint64_t span = (uint64_t)gridDim.x * blockDim.x * U;
-    for (uint64_t base = begin + (uint64_t)blockIdx.x * blockDim.x * U; base < n_all; base += span) {
+    const uint64_t span = (uint64_t)nblocks * blockDim.x * U;
+    for (uint64_t base = begin + (uint64_t)block * blockDim.x * U; base < n_all; base += span) {
         uint32_t t[U], c[U], r[U];
         bool alive[U];
 #pragma unroll
@@ -1160,6 +1179,12 @@ __global__ void k_count(WorldView<R> w, int all)
     }
 }
 
+template <class R>
+__global__ void k_count(WorldView<R> w)
+{
+    count_slots(w, 0u, blockIdx.x, gridDim.x);
+}
+
 // Classes of the simulators that were in the cells of TPB consecutive tiles of
 // the previous sort (one block per TPB tiles), in windows of kCountWindow
 // slots.  The rank within (old cell, class) follows the order of the slots:
@@ -1169,10 +1194,11 @@ __global__ void k_count(WorldView<R> w, int all)
 // from window to window.  Class 7 takes its rank from the device atomics.
 // 512-slot windows (two entries per thread) measured faster than 256, 1024
 // (1.18 against 1.21 and 1.28 ms on 1e8 simulators); 2048 spills.
+// The blocks past the first ntb count the step's inflow and clones.
 constexpr uint32_t kCountWindow = 512;
 
 template <class R, int Block, int TPB>
-__global__ void __launch_bounds__(Block) __attribute__((amdgpu_waves_per_eu(7))) k_count_tiles(WorldView<R> w)
+__global__ void __launch_bounds__(Block) __attribute__((amdgpu_waves_per_eu(7))) k_count_tiles(WorldView<R> w, uint32_t ntb)
 {
     constexpr int U = kCountWindow / Block;
     constexpr uint32_t kChunks = kCountWindow / 64;
@@ -1185,12 +1211,16 @@ __global__ void __launch_bounds__(Block) __attribute__((amdgpu_waves_per_eu(7)))
     __shared__ uint32_t s_cnt[kCells * 7];
     __shared__ uint32_t s_first[kChunks], s_last[kChunks], s_whole[kChunks];
     __shared__ uint32_t s_lastn[kChunks * 7], s_carry[kChunks * 7];
+    if (blockIdx.x >= ntb) {
+        count_slots(w, w.st->n, blockIdx.x - ntb, gridDim.x - ntb);
+        return;
+    }
     const uint32_t ntiles = w.st->ntiles;
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const unsigned long long below = (1ull << lane) - 1ull;
     // the grid is sized for the largest tile table; blocks stride over the
     // groups of this step's tiles
-    for (uint32_t t0 = blockIdx.x * (uint32_t)TPB; t0 < ntiles; t0 += gridDim.x * (uint32_t)TPB) {
+    for (uint32_t t0 = blockIdx.x * (uint32_t)TPB; t0 < ntiles; t0 += ntb * (uint32_t)TPB) {
     const uint32_t t1 = min(t0 + (uint32_t)TPB, ntiles);
     const uint32_t c0 = w.tile_first[t0];
     const uint32_t nct = w.tile_first[t1] - c0;
@@ -1321,12 +1351,16 @@ __global__ void __launch_bounds__(Block) __attribute__((amdgpu_waves_per_eu(7)))
 }
 
 // Per cell: population (stayers, arrivals through each distinct neighbour,
-// class 7) and the start of each class within the cell.
+// class 7) and the start of each class within the cell; per block of
+// kScanBlock cells (a thread each) the sum of the populations, for the
+// offsets.
 template <class R>
-__global__ void k_gather(WorldView<R> w)
+__global__ void __launch_bounds__(kScanBlock) k_gather(WorldView<R> w)
 {
     const uint32_t nc = (uint32_t)w.nc;
-    for (uint32_t d = blockIdx.x * blockDim.x + threadIdx.x; d < nc; d += gridDim.x * blockDim.x) {
+    const uint32_t d = blockIdx.x * kScanBlock + threadIdx.x;
+    uint32_t pop = 0u;
+    if (d < nc) {
         const size_t fb = (size_t)d * kMaxFaces;
         int32_t nb[kMaxFaces];
 #pragma unroll
@@ -1362,22 +1396,22 @@ __global__ void k_gather(WorldView<R> w)
             total += num[k];
         }
         pre[7] = total;
-        w.cnt[d] = total + w.ocnt[d];
+        pop = total + w.ocnt[d];
+        w.cnt[d] = pop;
+    }
+    __shared__ uint32_t sh[kScanBlock / 64];
+    const uint32_t inc = wave_incl_scan_u32(pop);
+    if ((threadIdx.x & 63u) == 63u) sh[threadIdx.x >> 6] = inc;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        uint32_t t = 0;
+#pragma unroll
+        for (int q = 0; q < kScanBlock / 64; ++q) t += sh[q];
+        w.blocksum[blockIdx.x] = t;
     }
 }
 
 // --------------------------------------------------------------- scan
-
-__device__ inline uint32_t wave_incl_scan_u32(uint32_t v)
-{
-    const int lane = (int)__lane_id();
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const uint32_t u = __shfl_up(v, o);
-        if (lane >= o) v += u;
-    }
-    return v;
-}
 
 // Block sums of kScanBlock-entry blocks (256 threads, four entries each).
 __global__ void k_scan_reduce(const uint32_t* in, uint32_t n, uint32_t* bsum)
@@ -1422,8 +1456,31 @@ __global__ void k_scan_bsum(uint32_t* bsum, uint32_t nb)
     }
 }
 
+// Where a block of a scan takes its base from: the scanned block sums, the
+// block sums before it (it adds them up itself), or the input before it.
+enum ScanBase { kBaseScanned = 0, kBaseSums = 1, kBaseInput = 2 };
+
+// Base of this block (256 threads, called by all of them).
+__device__ inline uint32_t scan_base(const uint32_t* in, const uint32_t* bsum, int from)
+{
+    if (from == kBaseScanned) return bsum[blockIdx.x];
+    __shared__ uint32_t sh[kBlock / 64];
+    const uint32_t* p = (from == kBaseSums) ? bsum : in;
+    const uint32_t m = (from == kBaseSums) ? blockIdx.x : blockIdx.x * kScanBlock;
+    uint32_t s = 0u;
+    for (uint32_t i = threadIdx.x; i < m; i += kBlock) s += p[i];
+    s = wave_incl_scan_u32(s);
+    if ((threadIdx.x & 63u) == 63u) sh[threadIdx.x >> 6] = s;
+    __syncthreads();
+    s = 0u;
+#pragma unroll
+    for (int q = 0; q < kBlock / 64; ++q) s += sh[q];
+    return s;
+}
+
 // Exclusive scan of in[0..n) into out; out[n-1] is the total when in[n-1]==0.
-__global__ void k_scan_apply(const uint32_t* in, uint32_t n, const uint32_t* bsum, uint32_t* out, uint32_t* total_out)
+__global__ void k_scan_apply(const uint32_t* in, uint32_t n, const uint32_t* bsum, uint32_t* out, uint32_t* total_out,
+                             int from)
 {
     __shared__ uint32_t sh[kBlock / 64];
     const uint32_t wv = threadIdx.x >> 6;
@@ -1433,8 +1490,8 @@ __global__ void k_scan_apply(const uint32_t* in, uint32_t n, const uint32_t* bsu
     for (int k = 0; k < 4; ++k) { v[k] = (b + k < n) ? in[b + k] : 0u; s += v[k]; }
     const uint32_t inc = wave_incl_scan_u32(s);
     if ((threadIdx.x & 63u) == 63u) sh[wv] = inc;
+    uint32_t run = scan_base(in, bsum, from) + inc - s;
     __syncthreads();
-    uint32_t run = bsum[blockIdx.x] + inc - s;
     for (uint32_t q = 0; q < wv; ++q) run += sh[q];
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
@@ -1446,26 +1503,85 @@ __global__ void k_scan_apply(const uint32_t* in, uint32_t n, const uint32_t* bsu
     }
 }
 
-// Exclusive scan of in[0..n) into out.  bsum holds scan_bsum_words(n) words:
-// the nb block sums, and past them, when nb exceeds kScanDirect, the sums of
-// the block sums (scanned in blocks themselves, as a single block scanning
-// many sums is slow).
+// Scans of more than kScanDirect blocks scan their block sums first (in one
+// block, or in blocks when they are many: a single block scanning many sums is
+// slow); below it every block adds the sums before it itself (at 4096 blocks
+// 33 MB of reads from L2, 5 us), which saves a launch; up to kScanInput blocks
+// read the input before them instead, which saves the sums too.
 constexpr uint32_t kScanDirect = 4096;
+constexpr uint32_t kScanInput = 16;
 
+// The nb block sums made ready for the blocks of a scan; returns their form.
+static int scan_block_sums(uint32_t* bsum, uint32_t nb, hipStream_t s)
+{
+    if (nb <= kScanDirect) return kBaseSums;
+    uint32_t* b2 = bsum + nb + 1;
+    const uint32_t nb2 = (nb + kScanBlock - 1) / kScanBlock;
+    hipLaunchKernelGGL(k_scan_reduce, dim3(nb2), dim3(kBlock), 0, s, bsum, nb, b2);
+    hipLaunchKernelGGL(k_scan_bsum, dim3(1), dim3(1024), 0, s, b2, nb2);
+    hipLaunchKernelGGL(k_scan_apply, dim3(nb2), dim3(kBlock), 0, s, bsum, nb, b2, bsum, nullptr, kBaseScanned);
+    return kBaseScanned;
+}
+
+// Exclusive scan of in[0..n) into out.  bsum holds scan_bsum_words(n) words:
+// the nb block sums, and past them the sums of the block sums.
 static void scan_u32(const uint32_t* in, uint32_t n, uint32_t* out, uint32_t* bsum, uint32_t* total, hipStream_t s)
 {
     const uint32_t nb = (n + kScanBlock - 1) / kScanBlock;
-    hipLaunchKernelGGL(k_scan_reduce, dim3(nb), dim3(kBlock), 0, s, in, n, bsum);
-    if (nb > kScanDirect) {
-        uint32_t* b2 = bsum + nb + 1;
-        const uint32_t nb2 = (nb + kScanBlock - 1) / kScanBlock;
-        hipLaunchKernelGGL(k_scan_reduce, dim3(nb2), dim3(kBlock), 0, s, bsum, nb, b2);
-        hipLaunchKernelGGL(k_scan_bsum, dim3(1), dim3(1024), 0, s, b2, nb2);
-        hipLaunchKernelGGL(k_scan_apply, dim3(nb2), dim3(kBlock), 0, s, bsum, nb, b2, bsum, nullptr);
-    } else {
-        hipLaunchKernelGGL(k_scan_bsum, dim3(1), dim3(1024), 0, s, bsum, nb);
+    int from = kBaseInput;
+    if (nb > kScanInput || in == out) {   // (blocks overwrite the input of a scan in place)
+        hipLaunchKernelGGL(k_scan_reduce, dim3(nb), dim3(kBlock), 0, s, in, n, bsum);
+        from = scan_block_sums(bsum, nb, s);
     }
-    hipLaunchKernelGGL(k_scan_apply, dim3(nb), dim3(kBlock), 0, s, in, n, bsum, out, total);
+    hipLaunchKernelGGL(k_scan_apply, dim3(nb), dim3(kBlock), 0, s, in, n, bsum, out, total, from);
+}
+
+// Cell offsets from the populations and k_gather's block sums, and the tile
+// table of the cell tiles with windows of 2^shift keys: tile_first[t] = first
+// cell whose key off[c] + kCellW * c is >= t << shift; tile_first[ntiles] =
+// nc.  Each cell writes the tiles that start at it.
+template <class R>
+__global__ void k_offsets(WorldView<R> w, int from, uint32_t shift)
+{
+    __shared__ uint32_t sh[kBlock / 64];
+    const uint32_t nc = (uint32_t)w.nc, wv = threadIdx.x >> 6;
+    const uint32_t b = blockIdx.x * kScanBlock + threadIdx.x * 4;
+    uint32_t v[4], s = 0;
+    int32_t ci[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        v[k] = (b + k < nc) ? w.cnt[b + k] : 0u;
+        ci[k] = (b + k < nc) ? w.cell_case[b + k] : 0;
+        s += v[k];
+    }
+    uint32_t before = (b > 0u && b <= nc) ? w.cnt[b - 1u] : 0u;   // population of the cell before
+    const uint32_t inc = wave_incl_scan_u32(s);
+    if ((threadIdx.x & 63u) == 63u) sh[wv] = inc;
+    uint32_t run = scan_base(w.cnt, w.blocksum, from) + inc - s;
+    __syncthreads();
+    for (uint32_t q = 0; q < wv; ++q) run += sh[q];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const uint32_t c = b + (uint32_t)k;
+        if (c <= nc) {
+            w.off[c] = run;
+            const uint64_t key = (uint64_t)run + (uint64_t)kCellW * c;
+            const uint64_t lo = (c == 0u) ? 0ull : (((uint64_t)(run - before) + (uint64_t)kCellW * (c - 1u)) >> shift) + 1ull;
+            uint64_t hi = key >> shift;
+            if (c == nc) {
+                hi += 1ull;
+                w.st->ntiles = (uint32_t)hi;
+                w.st->n_new = run;
+            }
+            for (uint64_t t = lo; t <= hi; ++t) {
+                w.tile_first[t] = c;
+                w.tile_p0[t] = run;
+                w.tile_case[t] = ci[k];
+            }
+        }
+        before = v[k];
+        run += v[k];
+    }
 }
 
 // ------------------------------------------------------------ scatter
@@ -1834,35 +1950,9 @@ __device__ inline void tile_sums(const WorldView<R>& w, uint32_t c0, uint32_t nc
     }
 }
 
-// ------------------------------------------------------------ tile table
-
-// tile_first[t] = first cell whose key off[c] + kCellW * c is >= t * TileN;
-// tile_first[ntiles] = nc.  Each cell writes the tiles that start at it.
-template <class R, uint32_t TileN>
-__global__ void k_tile_table(WorldView<R> w)
-{
-    const uint32_t nc = (uint32_t)w.nc;
-    for (uint32_t c = blockIdx.x * blockDim.x + threadIdx.x; c <= nc; c += gridDim.x * blockDim.x) {
-        const uint64_t key = (uint64_t)w.off[c] + (uint64_t)kCellW * c;
-        const uint64_t lo = (c == 0u) ? 0ull : ((uint64_t)w.off[c - 1] + (uint64_t)kCellW * (c - 1u)) / TileN + 1ull;
-        uint64_t hi = key / TileN;
-        if (c == nc) {
-            hi += 1ull;
-            w.st->ntiles = (uint32_t)hi;
-        }
-        const uint32_t p = w.off[c];
-        const int32_t ci = (c < nc) ? w.cell_case[c] : 0;
-        for (uint64_t t = lo; t <= hi; ++t) {
-            w.tile_first[t] = c;
-            w.tile_p0[t] = p;
-            w.tile_case[t] = ci;
-        }
-    }
-}
-
 // ------------------------------------------------------------ cell tiles
 
-// One block per tile (k_tile_table).  Steps:
+// One block per tile (k_offsets' table).  Steps:
 //  1. each cell's slot list (written by k_scatter in atomic order) is put in
 //     ascending previous-slot order: an entry's rank in its cell is the
 //     number of entries of that cell with a smaller slot;
@@ -3065,16 +3155,6 @@ __device__ inline bool kn_due(const CaseDev& cs)
            && ((cs.step + 1u) % (uint32_t)cs.decomposition_interval) == 0u;
 }
 
-template <class R>
-__global__ void k_kn_begin(WorldView<R> w)
-{
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c < w.ncases) {
-        CaseDev& cs = w.cases[c];
-        if (cs.active && cs.coll_model == UGX_COLL_HYBRID) cs.kn_time += cs.dt;
-    }
-}
-
 // kw[8c + 0..6] = rhoN, rhoM, p, T, U (localKnudsen.C:243-279)
 template <class R>
 __global__ void k_kn_fields(WorldView<R> w)
@@ -3648,9 +3728,7 @@ template void launch_nb_fill<double>(const WorldView<double>&, const uint32_t*, 
 template <class R, int Block, uint32_t TileN, uint32_t TileMax>
 static void launch_tiles_cfg(const WorldView<R>& w, hipStream_t s, bool sort_only)
 {
-    const uint32_t ncp = (uint32_t)w.nc + 1u;
     const unsigned nt = (unsigned)((w.cap + (uint64_t)kCellW * (uint64_t)w.nc) / TileN + 2);
-    hipLaunchKernelGGL((k_tile_table<R, TileN>), dim3(grid_for(ncp)), dim3(kBlock), 0, s, w);
     // species slots of the sums: 1 (single-species cases), 2, or all kNS
     const int nsl = (w.ns_max <= 1) ? 1 : (w.ns_max <= 2) ? 2 : kNS;
 #define UGX_TILE(SO, L, NS) hipLaunchKernelGGL((k_tile<R, SO, L, NS, Block, TileN, TileMax>), dim3(nt), dim3(Block), 0, s, w)
@@ -3676,17 +3754,28 @@ static void launch_tiles(const WorldView<R>& w, hipStream_t s, bool sort_only)
     }
 }
 
+// log2 of the key window of the current tile configuration.
+static uint32_t tile_shift(int variant) { return variant == 1 ? 9u : variant == 2 ? 7u : 8u; }
+
+// Cell populations, offsets and the tile table.
+template <class R>
+static void launch_offsets(const WorldView<R>& w, hipStream_t s)
+{
+    const uint32_t nb = ((uint32_t)w.nc + 1u + kScanBlock - 1) / kScanBlock;
+    hipLaunchKernelGGL(k_gather<R>, dim3(nb), dim3(kScanBlock), 0, s, w);
+    const int from = scan_block_sums(w.blocksum, nb, s);
+    hipLaunchKernelGGL(k_offsets<R>, dim3(nb), dim3(kBlock), 0, s, w, from, tile_shift(w.tile_variant));
+}
+
 template <class R>
 void launch_sort(const WorldView<R>& w, hipStream_t s)
 {
     const uint32_t ncp = (uint32_t)w.nc + 1u;
     const uint32_t n7 = (uint32_t)w.nc * 7u;
-    hipLaunchKernelGGL(k_zero_u32, dim3(grid_for(ncp)), dim3(kBlock), 0, s, w.cnt, ncp);
     hipLaunchKernelGGL(k_zero_u32, dim3(grid_for(ncp)), dim3(kBlock), 0, s, w.ocnt, ncp);
     hipLaunchKernelGGL(k_zero_u32, dim3(grid_for(n7)), dim3(kBlock), 0, s, w.out7, n7);
-    hipLaunchKernelGGL(k_count<R>, dim3(count_grid(w.cap)), dim3(kBlock), 0, s, w, 1);
-    hipLaunchKernelGGL(k_gather<R>, dim3(grid_for(w.nc)), dim3(kBlock), 0, s, w);
-    scan_u32(w.cnt, ncp, w.off, w.blocksum, &w.st->n_new, s);
+    hipLaunchKernelGGL(k_count<R>, dim3(count_grid(w.cap)), dim3(kBlock), 0, s, w);
+    launch_offsets<R>(w, s);
     hipLaunchKernelGGL(k_scatter<R>, dim3(count_grid(w.cap)), dim3(kBlock), 0, s, w);
     launch_tiles<R>(w, s, true);
     hipLaunchKernelGGL(k_finish_sort<R>, dim3(1), dim3(1), 0, s, w);
@@ -3711,27 +3800,20 @@ void launch_step(const WorldView<R>& w0, hipStream_t s, hipEvent_t* marks)
     const unsigned gc = grid_for((uint64_t)w.ncases);
     auto mark = [&](int i) { if (marks) (void)hipEventRecord(marks[i], s); };
     mark(0);
-    hipLaunchKernelGGL(k_begin_step<R>, dim3(gc), dim3(kBlock), 0, s, w);
-    hipLaunchKernelGGL(k_zero_u32, dim3(grid_for(ncp)), dim3(kBlock), 0, s, w.cnt, ncp);
-    hipLaunchKernelGGL(k_zero_u32, dim3(grid_for(ncp)), dim3(kBlock), 0, s, w.ocnt, ncp);
-    if (w.nwf > 0)
-        hipLaunchKernelGGL(k_zero_u32, dim3(grid_for((uint64_t)w.nwf + 1)), dim3(kBlock), 0, s, w.wcnt, (uint32_t)w.nwf + 1u);
+    hipLaunchKernelGGL(k_begin_step<R>, dim3(grid_for(std::max(ncp, (uint32_t)w.nwf + 1u) / 4u + 1u, 1024u)),
+                       dim3(kBeginBlock), 0, s, w);
     mark(1);
-    if (w.n_inflow > 0) {
-        if (w.n_inflow > 4096) {
-            // many inflow faces: counted in parallel and scanned in place
-            hipLaunchKernelGGL(k_inflow_face_count<R>, dim3(grid_for((uint64_t)w.n_inflow + 1)), dim3(kBlock), 0, s, w);
-            scan_u32(w.ins_off, (uint32_t)w.n_inflow + 1u, w.ins_off, w.blocksum, nullptr, s);
-            hipLaunchKernelGGL(k_inflow_finish<R>, dim3(1), dim3(1), 0, s, w);
-        } else {
-            hipLaunchKernelGGL(k_inflow_count<R>, dim3(1), dim3(1024), 0, s, w);
-        }
-        hipLaunchKernelGGL(k_inflow_gen<R>, dim3(grid_for(w.max_ins)), dim3(kBlock), 0, s, w);
+    if (w.n_inflow > kInflowBlock) {
+        // many inflow faces: counted in parallel and scanned in place
+        hipLaunchKernelGGL(k_inflow_face_count<R>, dim3(grid_for((uint64_t)w.n_inflow + 1)), dim3(kBlock), 0, s, w);
+        scan_u32(w.ins_off, (uint32_t)w.n_inflow + 1u, w.ins_off, w.blocksum, nullptr, s);
+        hipLaunchKernelGGL(k_inflow_finish<R>, dim3(1), dim3(1), 0, s, w);
     }
     mark(2);
     hipLaunchKernelGGL(k_move<R>, dim3(w.move_grid), dim3(kBlock), 0, s, w);
     mark(3);
-    hipLaunchKernelGGL(k_wall<R>, dim3(grid_for(w.wq_cap, 2048)), dim3(kBlock), 0, s, w);
+    const unsigned gwall = grid_for(w.wq_cap, 2048), gins = w.n_inflow > 0 ? grid_for(w.max_ins) : 0u;
+    hipLaunchKernelGGL(k_wall<R>, dim3(gwall + gins), dim3(kBlock), 0, s, w, gwall);
     if (w.nwf > 0) {
         const uint32_t nw1 = (uint32_t)w.nwf + 1u;
         scan_u32(w.wcnt, nw1, w.woff, w.blocksum, nullptr, s);
@@ -3750,16 +3832,14 @@ void launch_step(const WorldView<R>& w0, hipStream_t s, hipEvent_t* marks)
         hipLaunchKernelGGL(k_clone_finish<R>, dim3(1), dim3(64), 0, s, w);
     }
     mark(4);
-    hipLaunchKernelGGL((k_count_tiles<R, 256, kCountTiles>),
-                       dim3((unsigned)std::min<uint64_t>((max_tiles(w.cap, (uint64_t)w.nc) + kCountTiles - 1) / kCountTiles, kCountGrid)),
-                       dim3(256), 0, s, w);
-    // the slots past the existing simulators; a step's clones are few, so the
-    // grid is not sized for the bound
-    if (w.has_weighting || w.n_inflow > 0)
-        hipLaunchKernelGGL(k_count<R>, dim3(w.has_weighting ? 512u : grid_for(((uint64_t)w.max_ins + kCountUnroll - 1) / kCountUnroll, 512u)),
-                           dim3(kBlock), 0, s, w, 0);
-    hipLaunchKernelGGL(k_gather<R>, dim3(grid_for(w.nc)), dim3(kBlock), 0, s, w);
-    scan_u32(w.cnt, ncp, w.off, w.blocksum, &w.st->n_new, s);
+    // the slots past the existing simulators (a step's clones are few: their
+    // blocks are not sized for the bound) are counted beside the tiles
+    const unsigned gct = (unsigned)std::min<uint64_t>(
+        (max_tiles(w.cap, (uint64_t)w.nc) + kCountTiles - 1) / kCountTiles, kCountGrid);
+    const unsigned gcn = w.has_weighting ? 512u
+                         : w.n_inflow > 0 ? grid_for(((uint64_t)w.max_ins + kCountUnroll - 1) / kCountUnroll, 512u) : 0u;
+    hipLaunchKernelGGL((k_count_tiles<R, 256, kCountTiles>), dim3(gct + gcn), dim3(256), 0, s, w, gct);
+    launch_offsets<R>(w, s);
     mark(5);
     hipLaunchKernelGGL(k_scatter<R>, dim3(count_grid(w.cap)), dim3(kBlock), 0, s, w);
     mark(6);
@@ -3785,7 +3865,6 @@ void launch_step(const WorldView<R>& w0, hipStream_t s, hipEvent_t* marks)
         }
     }
     if (w.has_hybrid) {
-        hipLaunchKernelGGL(k_kn_begin<R>, dim3(gc), dim3(kBlock), 0, s, w);
         if (w.kn_due) launch_decompose<R>(w, s);
     }
     mark(8);
