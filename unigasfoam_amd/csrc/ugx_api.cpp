@@ -485,7 +485,7 @@ int ugx_tile_config(ugx_case* c, int32_t* variant, int32_t* threads, int32_t* wi
     UGX_GUARD_BEGIN
     CHECK_CASE(c);
     const World* w = c->world;
-    static const int32_t cfg[kTileVariants][3] = {{128, 256, 512}, {256, 512, 1024}, {64, 128, 256}};
+    static const int32_t cfg[kTileVariants][3] = {{128, 256, 512}, {256, 512, 1024}, {64, 128, 256}, {256, 256, 0}};
     const int v = w->tile_variant;
     if (variant) *variant = v;
     if (threads) *threads = cfg[v][0];

@@ -1949,13 +1949,13 @@ __device__ inline void cell_partials(const WorldView<R>& w, const Acc& A, uint32
 struct TileCase {
     double dt;
     uint32_t step;
-    int32_t sample_interval, coll_model, bgk_model, active, ns, sampler_full, adaptive;
+    int32_t sample_interval, coll_model, bgk_model, active, ns, sampler_full, adaptive, sp_base;
 };
 
 __device__ inline TileCase tile_case_of(const CaseDev& c)
 {
     return TileCase{c.dt, c.step, c.sample_interval, c.coll_model, c.bgk_model, c.active, c.ns, c.sampler_full,
-                    c.adaptive};
+                    c.adaptive, c.sp_base};
 }
 
 // Sums of the cells of one tile, eight cells per wave (group g of lanes
@@ -2019,87 +2019,107 @@ __device__ inline bool samples_now(const TileCase& cs)
     return cs.active && ((cs.step + 1u) % (uint32_t)cs.sample_interval) == 0u;
 }
 
+// What the sums of a cell are needed for.
+struct SumUse {
+    bool sample, hybrid, bgk, adapt;
+    __device__ bool any() const { return sample || hybrid || bgk || adapt; }
+};
+
+__device__ inline SumUse sum_use(const TileCase& cs)
+{
+    SumUse u{false, false, false, false};
+    if (cs.active) {
+        u.sample = ((cs.step + 1u) % (uint32_t)cs.sample_interval) == 0u;
+        u.hybrid = cs.coll_model == UGX_COLL_HYBRID;
+        u.bgk = (cs.coll_model == UGX_COLL_BGK || u.hybrid) && cs.bgk_model != UGX_BGK_NONE;
+        u.adapt = cs.adaptive != 0;
+    }
+    return u;
+}
+
+// The totals S of cell c into the sampler, the time sums and the BGK moments;
+// every lane of the cell's group holds the totals and lane j stores its rows.
+// have: pre holds the cell's sampler rows.
+template <int L, int NS, class R>
+__device__ inline void store_sums(const WorldView<R>& w, uint32_t c, uint32_t j, const TileCase& cs, const SumUse& use,
+                                  const double (&S)[SumRows<L, NS>::kN], const SampPre& pre, bool have)
+{
+    constexpr bool MS = NS > 1;
+    constexpr int B = SumRows<L, NS>::kBase;
+    const double dt = cs.dt;
+    if (use.sample) {
+        int rows[5];
+        double v[5];
+        samp_lane_rows<L, NS>(j, cs.ns, cs.sampler_full != 0, rows);
+        samp_lane_values<L, NS>(j, S, v);
+        double* sc = &w.samp[(size_t)c * kNSamp];
+#pragma unroll
+        for (int i = 0; i < 5; ++i)
+            if (rows[i] >= 0) sc[rows[i]] = (have ? pre.v[i] : sc[rows[i]]) + dt * v[i];
+    }
+    // lane j of the group writes rows j, j + 8, j + 16 and species j
+    double v[3] = {0.0, 0.0, 0.0}, vsp = 0.0;
+#pragma unroll
+    for (int q = 0; q < B; ++q)
+        if ((uint32_t)(q & 7) == j) v[q >> 3] = S[q];
+    if constexpr (MS) {
+#pragma unroll
+        for (int q = 0; q < NS; ++q)
+            if ((uint32_t)q == j) vsp = S[B + q];
+    } else {
+        vsp = (j == 0u) ? S[UGX_S_N] : 0.0;
+    }
+    if (use.hybrid) {
+        double* ka = &w.knacc[(size_t)kKnRows * c];
+        ka[j] += dt * v[0];
+        if (MS || j == 0u) ka[8 + j] += dt * vsp;
+    }
+    if (use.adapt) {
+        // uniGasDynamicAdapter::adapt (uniGasDynamicAdapter.C:526-547): the
+        // cell measurements of every step, weighted by the time step
+        double* aa = &w.adacc[(size_t)kKnRows * c];
+        aa[j] += dt * v[0];
+        if (MS || j == 0u) aa[8 + j] += dt * vsp;
+    }
+    if (use.bgk) {
+        double* mo = &w.mom[(size_t)c * kNMom];
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            const uint32_t q = j + 8u * (uint32_t)i;
+            if (q < (uint32_t)UGX_S_BASE) mo[q] = v[i];
+        }
+        mo[UGX_S_SPECIES_N + j] = vsp;
+    }
+}
+
 template <int L, int NS, int Block, class R, class Acc>
 __device__ inline void tile_sums(const WorldView<R>& w, uint32_t c0, uint32_t nct, const uint32_t* s_off,
                                  const Acc& A, const int32_t* s_cc, const TileCase* s_tc, int case0,
                                  const SampPre& pre)
 {
-    constexpr bool MS = NS > 1;
-    constexpr int B = SumRows<L, NS>::kBase, NR = SumRows<L, NS>::kN;
+    constexpr int NR = SumRows<L, NS>::kN;
     const uint32_t tid = threadIdx.x;
     const uint32_t wv = tid >> 6, lane = tid & 63u, g = lane >> 3, j = lane & 7u;
     for (uint32_t kb = 0; kb < nct; kb += (Block / 64) * 8) {
         const uint32_t k = kb + wv * 8u + g;
         uint32_t b = 0, e = 0;
-        bool sample = false, hybrid = false, bgk = false, adapt = false;
-        double dt = 0.0;
+        SumUse use{false, false, false, false};
         const uint32_t c = c0 + k;
         TileCase cs{};
         if (k < nct) {
             const int ci = s_cc[k];
             cs = (ci == case0) ? *s_tc : tile_case_of(w.cases[ci]);
-            if (cs.active) {
-                sample = ((cs.step + 1u) % (uint32_t)cs.sample_interval) == 0u;
-                hybrid = cs.coll_model == UGX_COLL_HYBRID;
-                bgk = (cs.coll_model == UGX_COLL_BGK || hybrid) && cs.bgk_model != UGX_BGK_NONE;
-                adapt = cs.adaptive != 0;
-                if (sample || hybrid || bgk || adapt) { b = s_off[k]; e = s_off[k + 1]; }
-                dt = cs.dt;
-            }
+            use = sum_use(cs);
+            if (use.any()) { b = s_off[k]; e = s_off[k + 1]; }
         }
-        const bool need = sample || hybrid || bgk || adapt;
-        if (__ballot(need) == 0ull) continue;
+        if (__ballot(use.any()) == 0ull) continue;
         double S[NR];
 #pragma unroll
         for (int q = 0; q < NR; ++q) S[q] = 0.0;
         cell_partials<L, NS, R, Acc>(w, A, b + j, e, S);
 #pragma unroll
         for (int q = 0; q < NR; ++q) S[q] = group8_total(S[q]);
-        if (need && sample) {
-            // every lane of the group holds the totals; lane j updates its rows
-            int rows[5];
-            double v[5];
-            samp_lane_rows<L, NS>(j, cs.ns, cs.sampler_full != 0, rows);
-            samp_lane_values<L, NS>(j, S, v);
-            double* sc = &w.samp[(size_t)c * kNSamp];
-            const bool have = pre.valid && kb == 0u;
-#pragma unroll
-            for (int i = 0; i < 5; ++i)
-                if (rows[i] >= 0) sc[rows[i]] = (have ? pre.v[i] : sc[rows[i]]) + dt * v[i];
-        }
-        // lane j of the group writes rows j, j + 8, j + 16 and species j
-        double v[3] = {0.0, 0.0, 0.0}, vsp = 0.0;
-#pragma unroll
-        for (int q = 0; q < B; ++q)
-            if ((uint32_t)(q & 7) == j) v[q >> 3] = S[q];
-        if constexpr (MS) {
-#pragma unroll
-            for (int q = 0; q < NS; ++q)
-                if ((uint32_t)q == j) vsp = S[B + q];
-        } else {
-            vsp = (j == 0u) ? S[UGX_S_N] : 0.0;
-        }
-        if (need && hybrid) {
-            double* ka = &w.knacc[(size_t)kKnRows * c];
-            ka[j] += dt * v[0];
-            if (MS || j == 0u) ka[8 + j] += dt * vsp;
-        }
-        if (need && adapt) {
-            // uniGasDynamicAdapter::adapt (uniGasDynamicAdapter.C:526-547): the
-            // cell measurements of every step, weighted by the time step
-            double* aa = &w.adacc[(size_t)kKnRows * c];
-            aa[j] += dt * v[0];
-            if (MS || j == 0u) aa[8 + j] += dt * vsp;
-        }
-        if (need && bgk) {
-            double* mo = &w.mom[(size_t)c * kNMom];
-#pragma unroll
-            for (int i = 0; i < 3; ++i) {
-                const uint32_t q = j + 8u * (uint32_t)i;
-                if (q < (uint32_t)UGX_S_BASE) mo[q] = v[i];
-            }
-            mo[UGX_S_SPECIES_N + j] = vsp;
-        }
+        store_sums<L, NS, R>(w, c, j, cs, use, S, pre, pre.valid && kb == 0u);
     }
 }
 
@@ -2270,6 +2290,203 @@ __global__ void __launch_bounds__(Block) __attribute__((amdgpu_waves_per_eu((NS 
         GlobAcc<R> A{w.b, w.sp.local, w.perm};
         tile_sums<L, NS, Block, R>(w, c0, nct, s_off, A, s_cc, &s_tc, case0, SampPre{{0.0, 0.0, 0.0, 0.0, 0.0}, false});
     }
+}
+
+// The same three steps without tiles, for dense cells: there a tile holds one
+// cell, more than LDS takes, so that k_tile's gather waits for its slot list
+// and its sums run on eight lanes of its block.  Here
+//  k_order      puts the slot lists in order (eight lanes per cell, only the
+//               cells with simulators that the occupancy count did not lay out,
+//               and of those only the entries from the first such slot on),
+//  k_gather_all copies the records by the slot list, cells or not: every lane
+//               of the chip streams,
+//  k_cell_sums  adds up the sorted records, eight lanes per cell, kSumFlight
+//               records of a lane in flight.
+// The sums' second pass over 20 of a record's 36 bytes costs less than the
+// waiting (cylinder of 5e7, 625 per cell: 3595 us with tiles, 1252 = 139 + 757
+// + 356 without; expansion of 1.2e7, 50 per cell: 373 and 348; heat bath of
+// 3.6e5, 30 per cell and most of them to be merged: 25 and 52).  The tuner
+// takes this form where it is faster.
+// First of the entries [lo, hi) of p (ascending) that is not below v.
+__device__ inline uint32_t lower_slot(const uint32_t* p, uint32_t lo, uint32_t hi, uint32_t v)
+{
+    while (lo < hi) {
+        const uint32_t mid = (lo + hi) >> 1;
+        if (p[mid] < v) lo = mid + 1u; else hi = mid;
+    }
+    return lo;
+}
+
+// Largest reordering that the eight lanes of a cell do by themselves; a larger
+// one takes the wave.  The cells of a wave lie a grid apart, so that a row of
+// inflow cells, each with many new simulators to merge, is spread over the chip
+// (cylinder of 5e7: 350 us on eight lanes each, neighbouring cells together;
+// 139 like this).
+constexpr uint32_t kOrderGroup = 128;
+
+template <class R>
+__global__ void __launch_bounds__(kBlock) k_order(WorldView<R> w)
+{
+    const uint32_t lane = threadIdx.x & 63u, j = threadIdx.x & 7u;
+    const uint32_t c = (threadIdx.x >> 3) * gridDim.x + blockIdx.x;
+    const uint32_t oc = (c < (uint32_t)w.nc) ? w.ocnt[c] : 0u;
+    // entries [lo, eo) are in order, those of [eo, e) are to be merged in
+    uint32_t lo = 0u, eo = 0u, e = 0u;
+    if (oc != 0u) {
+        e = w.off[c + 1u];
+        eo = e - oc;
+        uint32_t first = 0xFFFFFFFFu;   // smallest slot of the entries from eo on
+        for (uint32_t q = eo + j; q < e; q += 8u) first = min(first, w.perm[q]);
+        first = min(first, (uint32_t)__shfl_xor((int)first, 1));
+        first = min(first, (uint32_t)__shfl_xor((int)first, 2));
+        first = min(first, (uint32_t)__shfl_xor((int)first, 4));
+        lo = lower_slot(w.perm, w.off[c], eo, first);
+    }
+    const bool big = e - lo > kOrderGroup;
+    if (oc != 0u && !big) {
+        for (uint32_t i = lo + j; i < e; i += 8u) {
+            const uint32_t slot = w.perm[i];
+            uint32_t r = (i < eo) ? i : lower_slot(w.perm, lo, eo, slot);
+            for (uint32_t q = eo; q < e; ++q) r += (w.perm[q] < slot) ? 1u : 0u;
+            w.scratch[r] = slot;
+        }
+    }
+    __threadfence_block();   // (a cell's lanes are in one wave)
+    if (oc != 0u && !big)
+        for (uint32_t i = lo + j; i < e; i += 8u) w.perm[i] = w.scratch[i];
+    // the sorted merge list goes to the destination's cell ids, which the gather
+    // writes afterwards
+    uint32_t* sorted = w.b.cell;
+    for (unsigned long long m = __ballot(big && j == 0u); m != 0ull; m &= m - 1ull) {
+        const int src = __ffsll(m) - 1;
+        const uint32_t l = __shfl(lo, src), o = __shfl(eo, src), z = __shfl(e, src);
+        for (uint32_t i = o + lane; i < z; i += 64u) {
+            const uint32_t slot = w.perm[i];
+            uint32_t r = o;
+            for (uint32_t q = o; q < z; ++q) r += (w.perm[q] < slot) ? 1u : 0u;
+            sorted[r] = slot;
+        }
+        __threadfence_block();
+        for (uint32_t i = l + lane; i < z; i += 64u) {
+            const bool in = i < o;
+            const uint32_t slot = in ? w.perm[i] : sorted[i];
+            const uint32_t k = in ? lower_slot(sorted, o, z, slot) - o : lower_slot(w.perm, l, o, slot) - o;
+            w.scratch[i + k] = slot;
+        }
+        __threadfence_block();
+        for (uint32_t i = l + lane; i < z; i += 64u) w.perm[i] = w.scratch[i];
+    }
+}
+
+// Records of a thread in flight (2 and 8 are within 4%).  Ranges of slots per XCD
+// instead of round-robin blocks are slower (cylinder 757 us, 826).
+constexpr int kGatherUnroll = 4;
+
+template <class R>
+__global__ void __launch_bounds__(kBlock) k_gather_all(WorldView<R> w)
+{
+    constexpr int U = kGatherUnroll;
+    const uint32_t n = w.st->n_new;
+    const uint64_t span = (uint64_t)gridDim.x * kBlock * U;
+    for (uint64_t base = (uint64_t)blockIdx.x * kBlock * U; base < n; base += span) {
+        uint32_t t[U];
+        R x[U], y[U], z[U], vx[U], vy[U], vz[U], er[U];
+        uint32_t c[U], g[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const uint64_t i = base + (uint64_t)u * kBlock + threadIdx.x;
+            t[u] = w.perm[min(i, (uint64_t)n - 1u)];
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            x[u] = w.a.x[t[u]]; y[u] = w.a.y[t[u]]; z[u] = w.a.z[t[u]];
+            vx[u] = w.a.vx[t[u]]; vy[u] = w.a.vy[t[u]]; vz[u] = w.a.vz[t[u]];
+            er[u] = w.a.erot[t[u]];
+            c[u] = w.a.cell[t[u]];
+            g[u] = w.a.sp[t[u]];
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const uint64_t i = base + (uint64_t)u * kBlock + threadIdx.x;
+            if (i >= n) continue;
+            w.b.x[i] = x[u]; w.b.y[i] = y[u]; w.b.z[i] = z[u];
+            w.b.vx[i] = vx[u]; w.b.vy[i] = vy[u]; w.b.vz[i] = vz[u];
+            w.b.erot[i] = er[u];
+            w.b.cell[i] = c[u];
+            w.b.sp[i] = g[u];
+        }
+    }
+}
+
+constexpr int kSumFlight = 4;   // (cylinder 355 us; 2: 406, 8: 431)
+
+template <class R, int L, int NS>
+__global__ void __launch_bounds__(kBlock) k_cell_sums(WorldView<R> w)
+{
+    constexpr int NR = SumRows<L, NS>::kN, F = kSumFlight;
+    __shared__ TileCase s_tc;
+    __shared__ double s_spm[NS > 1 ? kLdsSpecies : 1];
+    __shared__ uint8_t s_spr[NS > 1 ? kLdsSpecies : 1], s_spl[NS > 1 ? kLdsSpecies : 1];
+    const uint32_t tid = threadIdx.x, j = tid & 7u, nc = (uint32_t)w.nc;
+    const uint32_t c0 = blockIdx.x * (kBlock / 8u), c = c0 + (tid >> 3);
+    uint32_t b = 0u, e = 0u;
+    const int case0 = w.cell_case[c0];
+    int ci = case0;
+    if (c < nc) {
+        b = w.off[c];
+        e = w.off[c + 1u];
+        ci = w.cell_case[c];
+    }
+    const bool lds_species = w.nsp <= (int)kLdsSpecies;
+    if (tid == 0u) s_tc = tile_case_of(w.cases[case0]);
+    if (NS > 1 && lds_species)
+        for (int g = (int)tid; g < w.nsp; g += kBlock) {
+            s_spm[g] = w.sp.mass[g];
+            s_spr[g] = (uint8_t)w.sp.rotdof[g];
+            s_spl[g] = (uint8_t)w.sp.local[g];
+        }
+    __syncthreads();
+    TileCase cs = s_tc;
+    if (ci != case0) cs = tile_case_of(w.cases[ci]);
+    SumUse use{false, false, false, false};
+    if (c < nc) use = sum_use(cs);
+    if (!use.any()) e = b;
+    if (__ballot(use.any()) == 0ull) return;
+    // a single-species case: its species' constants
+    const double m1 = (NS > 1) ? 0.0 : w.sp.mass[cs.sp_base];
+    const double rd1 = (NS > 1) ? 0.0 : (double)w.sp.rotdof[cs.sp_base];
+    double S[NR];
+#pragma unroll
+    for (int q = 0; q < NR; ++q) S[q] = 0.0;
+    auto pass = [&](uint32_t i, auto width) {
+        constexpr int W = decltype(width)::value;
+        uint32_t g[W];
+        R vx[W], vy[W], vz[W], er[W];
+#pragma unroll
+        for (int u = 0; u < W; ++u) {
+            const uint32_t k = i + 8u * u;
+            vx[u] = w.b.vx[k]; vy[u] = w.b.vy[k]; vz[u] = w.b.vz[k];
+            er[u] = w.b.erot[k];
+            g[u] = (NS > 1) ? w.b.sp[k] : 0u;
+        }
+#pragma unroll
+        for (int u = 0; u < W; ++u) {
+            double m = m1, rd = rd1;
+            int s = 0;
+            if constexpr (NS > 1) {
+                m = lds_species ? s_spm[g[u]] : w.sp.mass[g[u]];
+                rd = lds_species ? (double)s_spr[g[u]] : (double)w.sp.rotdof[g[u]];
+                s = lds_species ? (int)s_spl[g[u]] : w.sp.local[g[u]];
+            }
+            partial_add<L, NS>(m, (double)vx[u], (double)vy[u], (double)vz[u], (double)er[u], rd, s, S);
+        }
+    };
+    uint32_t i = b + j;
+    for (; i + 8u * (F - 1) < e; i += 8u * F) pass(i, std::integral_constant<int, F>{});
+    for (; i < e; i += 8u) pass(i, std::integral_constant<int, 1>{});
+#pragma unroll
+    for (int q = 0; q < NR; ++q) S[q] = group8_total(S[q]);
+    store_sums<L, NS, R>(w, c, j, cs, use, S, SampPre{{0.0, 0.0, 0.0, 0.0, 0.0}, false}, false);
 }
 
 // ------------------------------------------------------------- collisions
@@ -3895,14 +4112,32 @@ static void launch_tiles_cfg(const WorldView<R>& w, hipStream_t s, bool sort_onl
 #undef UGX_TILE
 }
 
-// Cell-tile configurations (threads, key window, LDS simulators); the
-// choice changes the speed only, never a result.
+template <class R>
+static void launch_cells(const WorldView<R>& w, hipStream_t s)
+{
+    const unsigned g = (unsigned)(((uint64_t)w.nc * 8u + kBlock - 1) / kBlock);
+    const int nsl = (w.ns_max <= 1) ? 1 : (w.ns_max <= 2) ? 2 : kNS;
+    hipLaunchKernelGGL(k_order<R>, dim3(g), dim3(kBlock), 0, s, w);
+    hipLaunchKernelGGL(k_gather_all<R>, dim3(grid_for((w.cap + kGatherUnroll - 1) / kGatherUnroll, 65536)), dim3(kBlock), 0, s, w);
+#define UGX_CELLS(L, NS) hipLaunchKernelGGL((k_cell_sums<R, L, NS>), dim3(g), dim3(kBlock), 0, s, w)
+#define UGX_CELLS_NS(L) \
+    do { if (nsl == 1) UGX_CELLS(L, 1); else if (nsl == 2) UGX_CELLS(L, 2); else UGX_CELLS(L, kNS); } while (0)
+    if (w.sum_level >= 2) UGX_CELLS_NS(2);
+    else if (w.sum_level == 1) UGX_CELLS_NS(1);
+    else UGX_CELLS_NS(0);
+#undef UGX_CELLS_NS
+#undef UGX_CELLS
+}
+
+// Cell-tile configurations (threads, key window, LDS simulators) and the form
+// without tiles; the choice changes the speed only, never a result.
 template <class R>
 static void launch_tiles(const WorldView<R>& w, hipStream_t s, bool sort_only)
 {
     switch (w.tile_variant) {
     case 1: launch_tiles_cfg<R, 256, 512, 1024>(w, s, sort_only); break;
     case 2: launch_tiles_cfg<R, 64, 128, 256>(w, s, sort_only); break;
+    case kTilesNone: if (!sort_only) { launch_cells<R>(w, s); break; } [[fallthrough]];
     default: launch_tiles_cfg<R, 128, 256, 512>(w, s, sort_only); break;
     }
 }

@@ -96,7 +96,7 @@ struct WorldView {
     uint32_t* perm;           // [cap]
     uint32_t* ins_off;        // [n_inflow+1]
     uint32_t* scratch;        // [cap] rank of each slot within its cell (count -> scatter), then
-                              //       the slot order of tiles larger than LDS
+                              //       the slot order of tiles larger than LDS and of k_order
     uint32_t* tile_first;     // [max tiles + 2] first cell of each tile
     uint32_t* tile_p0;        //                 its first sorted slot
     int32_t* tile_case;       //                 the case of its first cell
@@ -256,10 +256,12 @@ constexpr int kNMom = UGX_S_SPECIES_MCC;
 // of its last cell.
 // Tile configurations: (threads, TileN window, LDS simulators) =
 // (128, 256, 512), (256, 512, 1024), (64, 128, 256); the table is sized for
-// the smallest window.
+// the smallest window.  Configuration kTilesNone gathers and sums without
+// tiles (its table, for the occupancy count, has the first one's windows).
 constexpr uint32_t kCellW = 8;
 constexpr uint32_t kMinTileN = 128;
-constexpr int kTileVariants = 3;
+constexpr int kTileVariants = 4;
+constexpr int kTilesNone = 3;
 constexpr int kConsVariants = 2;
 constexpr uint32_t kLdsSpecies = 64;   // species tables up to this size are staged in LDS per tile
 inline uint64_t max_tiles(uint64_t cap, uint64_t nc) { return (cap + kCellW * nc) / kMinTileN + 2; }
