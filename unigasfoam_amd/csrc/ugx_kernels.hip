@@ -4352,6 +4352,29 @@ void launch_set_f64(double* d, double v, uint32_t n, hipStream_t s)
     hipLaunchKernelGGL(k_set_f64, dim3(grid_for(n)), dim3(kBlock), 0, s, d, v, n);
 }
 
+// Transposes the sampler rows of 64 cells per block through LDS: reads are one
+// contiguous stretch, writes 512-byte rows, which the link to the host takes as
+// whole lines.
+constexpr uint32_t kOutCells = 64;
+
+__global__ void __launch_bounds__(kBlock) k_samples_out(const double* samp, uint32_t n, double* out)
+{
+    __shared__ double s_rows[kOutCells * (kNSamp + 1)];
+    const uint32_t c0 = blockIdx.x * kOutCells, m = min(kOutCells, n - c0);
+    for (uint32_t i = threadIdx.x; i < m * kNSamp; i += kBlock)
+        s_rows[(i / kNSamp) * (kNSamp + 1) + i % kNSamp] = samp[(size_t)c0 * kNSamp + i];
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < kOutCells * kNSamp; i += kBlock) {
+        const uint32_t c = i % kOutCells, r = i / kOutCells;
+        if (c < m) out[(size_t)r * n + c0 + c] = s_rows[c * (kNSamp + 1) + r];
+    }
+}
+
+void launch_samples_out(const double* samp, uint32_t n, double* out, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_samples_out, dim3((n + kOutCells - 1) / kOutCells), dim3(kBlock), 0, s, samp, n, out);
+}
+
 __global__ void k_copy_probe(const float4* __restrict__ in, float4* __restrict__ out, size_t n)
 {
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) out[i] = in[i];

@@ -279,6 +279,8 @@ template <class R> void launch_fill(const WorldView<R>& w, hipStream_t s, int cc
                                     const double* nd, const double* T, double rotT, const double* U,
                                     int exact, const double* bblo, const double* bbhi,
                                     uint32_t* fill_cnt, uint32_t* fill_off, int ns, int ncell_case);
+// Sampler rows of n cells, cell-major in, row-major out (host or device memory).
+void launch_samples_out(const double* samp, uint32_t n, double* out, hipStream_t s);
 void launch_copy_probe(const void* in, void* out, size_t bytes, hipStream_t s);
 // Parameters of a meshFill: number densities per species, per-axis
 // temperatures and the drift velocity, stored into device memory at d

@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -245,6 +246,15 @@ struct World {
     std::vector<CaseDev> cases;          // host mirror (step advanced with the device)
     std::vector<CaseSpec> specs_host;
     std::vector<int64_t> samp_reset_steps;
+    // Sampler downloads: kStageSlots parts of pinned host memory, each with an
+    // event, sized for the largest case and at most kStageBytes in all.
+    static constexpr int kStageSlots = 4;
+    static constexpr size_t kStageBytes = size_t(16) << 20;
+    static constexpr size_t kStageThreadBytes = size_t(1) << 20;   // larger downloads are copied by several threads
+    std::mutex stage_mu;           // (cases of one world may be read by several threads)
+    double* h_stage = nullptr;
+    uint32_t stage_cells = 0;      // cells per slot
+    hipEvent_t stage_ev[kStageSlots] = {};
 
     ~World();
     void release();
