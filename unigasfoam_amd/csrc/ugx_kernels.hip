@@ -2898,91 +2898,6 @@ __global__ void __launch_bounds__(kBlock) k_collide(WorldView<R> w)
     case_add(w.counters, ccase, kCntBgk, (unsigned long long)nrel);
 }
 
-// New velocity of one selected simulator (slot i of cell c, selection k)
-// from the parameters P.
-template <class R>
-__device__ inline void bgk_draw_core(const WorldView<R>& w, const CaseDev& cs, uint32_t c, uint32_t i, uint32_t k,
-                                     const BgkP& P, unsigned long long* raise, const GlobAcc<R>& A)
-{
-    Rng rv;
-    rng_init(rv, cs.seed_lo, cs.seed_hi, kRngBgkV, k, c - (uint32_t)cs.cell_begin, cs.step);
-    // a single-species case needs no species lookup
-    const int ls = (cs.ns == 1) ? 0 : A.local_species(i);
-    const double u0 = P.s2kT / sqrt(w.sp.mass[cs.sp_base + ls]);
-    if constexpr (sizeof(R) == sizeof(float)) {
-        // FP32 state: the draw in single precision (the stored velocity is FP32)
-        float xf[3];
-        if (P.model == UGX_BGK_USP) {
-            const float m0 = (float)P.m0;
-            const float Af = (float)(P.cQ / (P.p * u0)), Bf = (float)(P.cS / P.p), inv_m0 = 1.0f / m0;
-            const float q0 = (float)P.q[0], q1 = (float)P.q[1], q2 = (float)P.q[2];
-            const float s0 = (float)P.sm[0], s1 = (float)P.sm[1], s2 = (float)P.sm[2], s3 = (float)P.sm[3],
-                        s4 = (float)P.sm[4], s5 = (float)P.sm[5];
-            for (int it = 0; it < 100000; ++it) {
-                float g0, g1, g2;
-                gauss3f(rv, g0, g1, g2);
-                xf[0] = g0 * (float)kSqrtHalf; xf[1] = g1 * (float)kSqrtHalf; xf[2] = g2 * (float)kSqrtHalf;
-                const float vSq = xf[0] * xf[0] + xf[1] * xf[1] + xf[2] * xf[2];
-                const float vTr = vSq * (float)kThird;
-                const float prob = 1.0f + Af * (q0 * xf[0] + q1 * xf[1] + q2 * xf[2]) * (vSq * 0.4f - 1.0f)
-                                   + Bf * (s0 * (xf[0] * xf[0] - vTr) + s3 * (xf[1] * xf[1] - vTr)
-                                           + s5 * (xf[2] * xf[2] - vTr) + 2.0f * s1 * xf[0] * xf[1]
-                                           + 2.0f * s2 * xf[0] * xf[2] + 2.0f * s4 * xf[1] * xf[2]);
-                if (prob > m0 && prob < 10.0f) {
-                    atomicMax(raise, (unsigned long long)double_to_bits((double)prob));
-                    break;
-                }
-                if (uniformf(rv) < prob * inv_m0) break;
-            }
-        } else {
-            float g0, g1, g2;
-            gauss3f(rv, g0, g1, g2);
-            xf[0] = g0 * (float)kSqrtHalf; xf[1] = g1 * (float)kSqrtHalf; xf[2] = g2 * (float)kSqrtHalf;
-            if (P.model == UGX_BGK_ESBGK) {
-                float y[3];
-                for (int d = 0; d < 3; ++d)
-                    y[d] = (float)P.sm[3 * d] * xf[0] + (float)P.sm[3 * d + 1] * xf[1] + (float)P.sm[3 * d + 2] * xf[2];
-                xf[0] = y[0]; xf[1] = y[1]; xf[2] = y[2];
-            }
-        }
-        A.store(i, P.U[0] + u0 * (double)xf[0], P.U[1] + u0 * (double)xf[1], P.U[2] + u0 * (double)xf[2]);
-        return;
-    }
-    double xi[3];
-    if (P.model == UGX_BGK_USP) {
-        // the draw's constants are divided out once (usp_draw of the oracle)
-        const double m0 = P.m0;
-        const double A = P.cQ / (P.p * u0), B = P.cS / P.p, inv_m0 = 1.0 / m0;
-        for (int it = 0; it < 100000; ++it) {
-            double g0, g1, g2;
-            gauss3(rv, g0, g1, g2);
-            xi[0] = g0 * kSqrtHalf; xi[1] = g1 * kSqrtHalf; xi[2] = g2 * kSqrtHalf;
-            const double vSq = xi[0] * xi[0] + xi[1] * xi[1] + xi[2] * xi[2];
-            const double vTr = vSq * kThird;
-            const double* sh = P.sm;
-            const double prob = 1.0 + A * (P.q[0] * xi[0] + P.q[1] * xi[1] + P.q[2] * xi[2]) * (vSq * 0.4 - 1.0)
-                                + B * (sh[0] * (xi[0] * xi[0] - vTr) + sh[3] * (xi[1] * xi[1] - vTr)
-                                       + sh[5] * (xi[2] * xi[2] - vTr) + 2.0 * sh[1] * xi[0] * xi[1]
-                                       + 2.0 * sh[2] * xi[0] * xi[2] + 2.0 * sh[4] * xi[1] * xi[2]);
-            if (prob > m0 && prob < 10.0) {
-                atomicMax(raise, (unsigned long long)double_to_bits(prob));
-                break;
-            }
-            if (uniform(rv) < prob * inv_m0) break;
-        }
-    } else {
-        double g0, g1, g2;
-        gauss3(rv, g0, g1, g2);
-        xi[0] = g0 * kSqrtHalf; xi[1] = g1 * kSqrtHalf; xi[2] = g2 * kSqrtHalf;
-        if (P.model == UGX_BGK_ESBGK) {
-            double y[3];
-            for (int d = 0; d < 3; ++d) y[d] = P.sm[3 * d] * xi[0] + P.sm[3 * d + 1] * xi[1] + P.sm[3 * d + 2] * xi[2];
-            xi[0] = y[0]; xi[1] = y[1]; xi[2] = y[2];
-        }
-    }
-    A.store(i, P.U[0] + u0 * xi[0], P.U[1] + u0 * xi[1], P.U[2] + u0 * xi[2]);
-}
-
 // interpolationCellPoint at position x (cell frame) of cell c: the tet of
 // the cell's decomposition (centroid, then per face the fan (p0, p_i,
 // p_i+1), faces in ascending order) that holds x, or the one x is least
@@ -3077,30 +2992,18 @@ __device__ inline void macro_params(const WorldView<R>& w, const CaseDev& cs, ui
     }
 }
 
-// Macro: the world has macroInterpolation cases (a separate instance keeps
-// the interpolation's registers out of the plain draws).
-template <class R, bool Macro>
-__device__ inline void bgk_draw(const WorldView<R>& w, const CaseDev& cs, uint32_t c, uint32_t i, uint32_t k,
-                                const BgkP& P, unsigned long long* raise, const GlobAcc<R>& A)
-{
-    if (Macro && cs.macro) {
-        BgkP Q = P;
-        macro_params<R>(w, cs, c, i, Q);
-        bgk_draw_core<R>(w, cs, c, i, k, Q, raise, A);
-    } else {
-        bgk_draw_core<R>(w, cs, c, i, k, P, raise, A);
-    }
-}
-
 // One selected simulator's draw held by a lane across its rejection trials
-// (the same stream and arithmetic as bgk_draw_core, one trial at a time).
+// (the selection's stream, kRngBgkV with sub = selection index).
 // T is the draw's precision: single for the FP32 state.  e0..e8 hold the USP
 // stress (xx xy xz yy yz zz) or the ES-BGK matrix (row major).  Scalar
 // members, not arrays, so that the state stays in registers.
 template <class R>
 struct DrawLane {
     using T = typename std::conditional<sizeof(R) == sizeof(float), float, double>::type;
-    Rng rv;
+    // the stream's next block and, before an odd trial, the number left over from
+    // the last block
+    uint32_t k0, k1, blk, id, step, kind;
+    uint64_t left;
     T m0, inv_m0, a, bq, q0, q1, q2, e0, e1, e2, e3, e4, e5, e6, e7, e8;
     double u0, U0, U1, U2;
     uint32_t i, cc;
@@ -3139,7 +3042,11 @@ __device__ __attribute__((always_inline)) inline void draw_setup(const WorldView
                                                                  const double* pre = nullptr)
 {
     using T = typename DrawLane<R>::T;
-    rng_init(D.rv, cs.seed_lo, cs.seed_hi, kRngBgkV, k, c - (uint32_t)cs.cell_begin, cs.step);
+    Rng rv;
+    rng_init(rv, cs.seed_lo, cs.seed_hi, kRngBgkV, k, c - (uint32_t)cs.cell_begin, cs.step);
+    D.k0 = rv.k0; D.k1 = rv.k1;
+    D.blk = rv.c0; D.id = rv.c1; D.step = rv.c2; D.kind = rv.c3;
+    D.left = 0ull;
     if (pre) {
         D.u0 = pre[0];
     } else {
@@ -3173,6 +3080,17 @@ __device__ __attribute__((always_inline)) inline void draw_setup(const WorldView
     }
 }
 
+// The stream's next block: two of its numbers.
+template <class R>
+__device__ __attribute__((always_inline)) inline void draw_block(DrawLane<R>& D, uint64_t& a, uint64_t& b)
+{
+    uint32_t c0 = D.blk, c1 = D.id, c2 = D.step, c3 = D.kind;
+    philox10(c0, c1, c2, c3, D.k0, D.k1);
+    D.blk += 1u;
+    a = ((uint64_t)c0 << 32) | c1;
+    b = ((uint64_t)c2 << 32) | c3;
+}
+
 // One trial: true when (x0, x1, x2) holds the drawn thermal velocity
 // (accepted, the only draw of the BGK and ES-BGK models, or the last
 // allowed USP trial).
@@ -3183,9 +3101,34 @@ __device__ __attribute__((always_inline)) inline bool draw_trial(DrawLane<R>& D,
                                                                  typename DrawLane<R>::T& x2)
 {
     using T = typename DrawLane<R>::T;
-    T g0, g1, g2;
-    if constexpr (sizeof(T) == sizeof(float)) gauss3f(D.rv, g0, g1, g2);
-    else gauss3(D.rv, g0, g1, g2);
+    // A trial takes an odd count of numbers (3 in single precision, 5 in double),
+    // so every second trial begins with the second number of a block.  The
+    // blocks are made at fixed places of the trial, the last one only for the
+    // even trials of the USP model: lanes at odd and at even trials then share
+    // them.  Drawing number by number ran a masked block at each number, twice
+    // as many (expansion of 1.2e7: draws and conservation 787 us, like this 668; in
+    // FP64, 1.6e6: 369 us, 320).
+    constexpr bool kSingle = sizeof(T) == sizeof(float);
+    const bool odd = (D.it & 1) != 0, usp = D.model == UGX_BGK_USP;
+    uint64_t n1, n2, n4;
+    T g0, g1, g2, g3;
+    draw_block<R>(D, n1, n2);
+    if constexpr (kSingle) {
+        // odd: left, n1 | n2; even: n1, n2 | next
+        const uint64_t u0 = odd ? D.left : n1, u1 = odd ? n1 : n2;
+        n4 = n2;
+        if (usp && !odd) draw_block<R>(D, n4, D.left);
+        gauss2f(u0, g0, g1);
+        gauss2f(u1, g2, g3);
+    } else {
+        uint64_t n3, n0;
+        draw_block<R>(D, n3, n0);
+        const uint64_t u0 = odd ? D.left : n1, u1 = odd ? n1 : n2, u2 = odd ? n2 : n3, u3 = odd ? n3 : n0;
+        n4 = n0;
+        if (usp && !odd) draw_block<R>(D, n4, D.left);
+        gauss2(u0, u1, g0, g1);
+        gauss2(u2, u3, g2, g3);
+    }
     x0 = g0 * (T)kSqrtHalf; x1 = g1 * (T)kSqrtHalf; x2 = g2 * (T)kSqrtHalf;
     if (D.model == UGX_BGK_USP) {
         const T vSq = x0 * x0 + x1 * x1 + x2 * x2;
@@ -3199,8 +3142,8 @@ __device__ __attribute__((always_inline)) inline bool draw_trial(DrawLane<R>& D,
             return true;
         }
         T u;
-        if constexpr (sizeof(T) == sizeof(float)) u = uniformf(D.rv);
-        else u = uniform(D.rv);
+        if constexpr (kSingle) u = uniform24_open0((uint32_t)(n4 >> 32));
+        else u = uniform(n4);
         if (u < prob * D.inv_m0) return true;
         D.it += 1;
         return D.it >= 100000;
