@@ -106,15 +106,51 @@ __host__ __device__ inline uint64_t rng_u64(Rng& r)
     return v;
 }
 
+// The next two and the next three numbers of the stream, with the blocks made
+// at fixed places: lanes that have a number left from their last block (half ==
+// 1) and lanes that have none share them.  Drawn one by one, each number would
+// run a masked block in a wave that holds both.
+__host__ __device__ inline void rng_block(Rng& r, uint64_t& a, uint64_t& b)
+{
+    uint32_t c0 = r.c0, c1 = r.c1, c2 = r.c2, c3 = r.c3;
+    philox10(c0, c1, c2, c3, r.k0, r.k1);
+    r.c0 += 1u;
+    a = ((uint64_t)c0 << 32) | c1;
+    b = ((uint64_t)c2 << 32) | c3;
+}
+
+__host__ __device__ inline void rng_u64x2(Rng& r, uint64_t& v0, uint64_t& v1)
+{
+    uint64_t a, b;
+    rng_block(r, a, b);
+    const bool left = r.half == 1;
+    v0 = left ? ((uint64_t)r.b2 << 32) | r.b3 : a;
+    v1 = left ? a : b;
+    if (left) { r.b2 = (uint32_t)(b >> 32); r.b3 = (uint32_t)b; }
+}
+
+__host__ __device__ inline void rng_u64x3(Rng& r, uint64_t& v0, uint64_t& v1, uint64_t& v2)
+{
+    rng_u64x2(r, v0, v1);
+    if (r.half == 1) {
+        v2 = ((uint64_t)r.b2 << 32) | r.b3;
+        r.half = 2;
+    } else {
+        uint64_t b;
+        rng_block(r, v2, b);
+        r.b2 = (uint32_t)(b >> 32);
+        r.b3 = (uint32_t)b;
+        r.half = 1;
+    }
+}
+
 // Uniform on (0, 1].
 __host__ __device__ inline double uniform(uint64_t v) { return (double)((v >> 11) + 1u) * 0x1.0p-53; }
 __host__ __device__ inline double uniform(Rng& r) { return uniform(rng_u64(r)); }
 
 // Uniform integer in [0, n).
-__host__ __device__ inline uint32_t uindex(Rng& r, uint32_t n)
-{
-    return (uint32_t)(((rng_u64(r) >> 32) * (uint64_t)n) >> 32);
-}
+__host__ __device__ inline uint32_t uindex(uint64_t v, uint32_t n) { return (uint32_t)(((v >> 32) * (uint64_t)n) >> 32); }
+__host__ __device__ inline uint32_t uindex(Rng& r, uint32_t n) { return uindex(rng_u64(r), n); }
 
 // ----------------------------------------------------- deterministic math
 // Cody-Waite reduction + truncated series; only +, -, *, /, floor.
@@ -243,8 +279,8 @@ __host__ __device__ inline void gauss2(uint64_t v1, uint64_t v2, double& g0, dou
 
 __host__ __device__ inline void gauss2(Rng& r, double& g0, double& g1)
 {
-    const uint64_t v1 = rng_u64(r);
-    const uint64_t v2 = rng_u64(r);
+    uint64_t v1, v2;
+    rng_u64x2(r, v1, v2);
     gauss2(v1, v2, g0, g1);
 }
 
@@ -631,10 +667,12 @@ __device__ inline void scatter(Rng& r, int vss, double alpha, double cR, const d
 {
     double Ucm[3];
     for (int d = 0; d < 3; ++d) Ucm[d] = (mP * UP[d] + mQ * UQ[d]) / (mP + mQ);
-    double cosT = vss ? 2.0 * dpow(uniform(r), 1.0 / alpha) - 1.0 : 2.0 * uniform(r) - 1.0;
+    uint64_t vT, vP;
+    rng_u64x2(r, vT, vP);
+    double cosT = vss ? 2.0 * dpow(uniform(vT), 1.0 / alpha) - 1.0 : 2.0 * uniform(vT) - 1.0;
     double sinT = sqrt(1.0 - cosT * cosT);
     double sp, cp;
-    dsincos2pi(uniform(r), sp, cp);
+    dsincos2pi(uniform(vP), sp, cp);
     double c[3];
     double D = sqrt(crc[1] * crc[1] + crc[2] * crc[2]);
     if (vss && D > 0.0) {
