@@ -491,7 +491,7 @@ int ugx_tile_config(ugx_case* c, int32_t* variant, int32_t* threads, int32_t* wi
     if (threads) *threads = cfg[v][0];
     if (window) *window = cfg[v][1];
     if (lds_simulators) *lds_simulators = cfg[v][2];
-    if (tuned) *tuned = (!w->autotune || w->tune_step >= kTileVariants) ? 1 : 0;
+    if (tuned) *tuned = (!w->autotune || w->tune_step >= World::kTuneSteps) ? 1 : 0;
     return UGX_OK;
     UGX_GUARD_END
 }

@@ -1131,10 +1131,46 @@ __global__ void k_clone_finish(WorldView<R> w)
 // do not depend on the order in which the hits were recorded
 // (uniGasPatchBoundary.C:130-302 measures in the order of the cloud's list).
 
+// Up to kWallScanFaces faces every block scans the counts itself (the first one
+// stores the offsets), which saves a launch (4.5 us of a channel's step of
+// 150); more faces (woff) are scanned before.
+constexpr int kWallScanFaces = 4096;
+
 template <class R>
-__global__ void k_wall_bucket(WorldView<R> w)
+__global__ void __launch_bounds__(kBlock) k_wall_bucket(WorldView<R> w)
 {
     const uint32_t n = w.st->nev;
+    if (w.nwf <= kWallScanFaces) {
+        __shared__ uint32_t s_off[kWallScanFaces + 1], sh[kBlock / 64];
+        if (blockIdx.x != 0u && blockIdx.x * kBlock >= n) return;
+        const uint32_t nf = (uint32_t)w.nwf, wv = threadIdx.x >> 6;
+        for (uint32_t i = threadIdx.x; i < nf; i += kBlock) s_off[i] = w.wcnt[i];
+        __syncthreads();
+        const uint32_t per = (nf + kBlock - 1u) / kBlock, lo = min(nf, threadIdx.x * per), hi = min(nf, lo + per);
+        uint32_t sum = 0u;
+        for (uint32_t i = lo; i < hi; ++i) sum += s_off[i];
+        const uint32_t inc = wave_incl_scan_u32(sum);
+        if ((threadIdx.x & 63u) == 63u) sh[wv] = inc;
+        __syncthreads();
+        uint32_t run = inc - sum;
+        for (uint32_t q = 0; q < wv; ++q) run += sh[q];
+        for (uint32_t i = lo; i < hi; ++i) {
+            const uint32_t v = s_off[i];
+            s_off[i] = run;
+            run += v;
+        }
+        if (threadIdx.x == kBlock - 1) s_off[nf] = run;
+        __syncthreads();
+        if (blockIdx.x == 0u)
+            for (uint32_t i = threadIdx.x; i <= nf; i += kBlock) w.woff[i] = s_off[i];
+        if (n > w.ev_cap) return;   // the step is in error (evover)
+        for (uint32_t i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) {
+            const uint32_t pos = s_off[w.ev[i].wf] + w.ev[i].rank;
+            w.bkey[pos] = w.ev_key[i];
+            w.bidx[pos] = i;
+        }
+        return;
+    }
     if (n > w.ev_cap) return;   // the step is in error (evover)
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
         const uint32_t pos = w.woff[w.ev[i].wf] + w.ev[i].rank;
@@ -1503,12 +1539,34 @@ __global__ void __launch_bounds__(Block) __attribute__((amdgpu_waves_per_eu(7)))
     }
 }
 
+// Offset `run` of cell c (c = nc: the end) after a cell of `before` simulators,
+// and the tiles of 2^shift keys that start at it (k_offsets).
+template <class R>
+__device__ inline void put_offset(const WorldView<R>& w, uint32_t c, uint32_t run, uint32_t before, int32_t ccase,
+                                  uint32_t shift)
+{
+    w.off[c] = run;
+    const uint64_t key = (uint64_t)run + (uint64_t)kCellW * c;
+    const uint64_t lo = (c == 0u) ? 0ull : (((uint64_t)(run - before) + (uint64_t)kCellW * (c - 1u)) >> shift) + 1ull;
+    uint64_t hi = key >> shift;
+    if (c == (uint32_t)w.nc) {
+        hi += 1ull;
+        w.st->ntiles = (uint32_t)hi;
+        w.st->n_new = run;
+    }
+    for (uint64_t t = lo; t <= hi; ++t) {
+        w.tile_first[t] = c;
+        w.tile_p0[t] = run;
+        w.tile_case[t] = ccase;
+    }
+}
+
 // Per cell: population (stayers, arrivals through each distinct neighbour,
 // class 7) and the start of each class within the cell; per block of
 // kScanBlock cells (a thread each) the sum of the populations, for the
 // offsets.
 template <class R>
-__global__ void __launch_bounds__(kScanBlock) k_gather(WorldView<R> w)
+__global__ void __launch_bounds__(kScanBlock) k_gather(WorldView<R> w, uint32_t shift)
 {
     const uint32_t nc = (uint32_t)w.nc;
     const uint32_t d = blockIdx.x * kScanBlock + threadIdx.x;
@@ -1556,6 +1614,17 @@ __global__ void __launch_bounds__(kScanBlock) k_gather(WorldView<R> w)
     const uint32_t inc = wave_incl_scan_u32(pop);
     if ((threadIdx.x & 63u) == 63u) sh[threadIdx.x >> 6] = inc;
     __syncthreads();
+    if (gridDim.x == 1u) {
+        // all cells are here: the offsets and the tile table too, which saves a launch
+        uint32_t run = inc - pop;
+        for (uint32_t q = 0; q < (threadIdx.x >> 6); ++q) run += sh[q];
+        __shared__ uint32_t s_pop[kScanBlock];
+        s_pop[threadIdx.x] = pop;
+        __syncthreads();
+        const uint32_t before = (d > 0u) ? s_pop[d - 1u] : 0u;
+        if (d <= nc) put_offset(w, d, run, before, (d < nc) ? w.cell_case[d] : 0, shift);
+        return;
+    }
     if (threadIdx.x == 0) {
         uint32_t t = 0;
 #pragma unroll
@@ -1716,22 +1785,7 @@ __global__ void k_offsets(WorldView<R> w, int from, uint32_t shift)
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
         const uint32_t c = b + (uint32_t)k;
-        if (c <= nc) {
-            w.off[c] = run;
-            const uint64_t key = (uint64_t)run + (uint64_t)kCellW * c;
-            const uint64_t lo = (c == 0u) ? 0ull : (((uint64_t)(run - before) + (uint64_t)kCellW * (c - 1u)) >> shift) + 1ull;
-            uint64_t hi = key >> shift;
-            if (c == nc) {
-                hi += 1ull;
-                w.st->ntiles = (uint32_t)hi;
-                w.st->n_new = run;
-            }
-            for (uint64_t t = lo; t <= hi; ++t) {
-                w.tile_first[t] = c;
-                w.tile_p0[t] = run;
-                w.tile_case[t] = ci[k];
-            }
-        }
+        if (c <= nc) put_offset(w, c, run, before, ci[k], shift);
         before = v[k];
         run += v[k];
     }
@@ -1996,8 +2050,7 @@ __device__ inline void samp_lane_values(uint32_t j, const double (&S)[NR], doubl
 #pragma unroll
     for (int i = 0; i < 5; ++i) v[i] = 0.0;
 #pragma unroll
-    for (int q = 0; q < B; ++q)
-        if ((uint32_t)(q & 7) == j) v[q >> 3] = S[q];
+    for (int q = 0; q < B; ++q) v[q >> 3] = ((uint32_t)(q & 7) == j) ? S[q] : v[q >> 3];
     if constexpr (MS) {
 #pragma unroll
         for (int q = 0; q < NS; ++q)
@@ -2041,7 +2094,7 @@ __device__ inline SumUse sum_use(const TileCase& cs)
 // every lane of the cell's group holds the totals and lane j stores its rows.
 // have: pre holds the cell's sampler rows.
 template <int L, int NS, class R>
-__device__ inline void store_sums(const WorldView<R>& w, uint32_t c, uint32_t j, const TileCase& cs, const SumUse& use,
+__device__ __attribute__((always_inline)) inline void store_sums(const WorldView<R>& w, uint32_t c, uint32_t j, const TileCase& cs, const SumUse& use,
                                   const double (&S)[SumRows<L, NS>::kN], const SampPre& pre, bool have)
 {
     constexpr bool MS = NS > 1;
@@ -2060,8 +2113,7 @@ __device__ inline void store_sums(const WorldView<R>& w, uint32_t c, uint32_t j,
     // lane j of the group writes rows j, j + 8, j + 16 and species j
     double v[3] = {0.0, 0.0, 0.0}, vsp = 0.0;
 #pragma unroll
-    for (int q = 0; q < B; ++q)
-        if ((uint32_t)(q & 7) == j) v[q >> 3] = S[q];
+    for (int q = 0; q < B; ++q) v[q >> 3] = ((uint32_t)(q & 7) == j) ? S[q] : v[q >> 3];
     if constexpr (MS) {
 #pragma unroll
         for (int q = 0; q < NS; ++q)
@@ -4122,9 +4174,11 @@ template <class R>
 static void launch_offsets(const WorldView<R>& w, hipStream_t s)
 {
     const uint32_t nb = ((uint32_t)w.nc + 1u + kScanBlock - 1) / kScanBlock;
-    hipLaunchKernelGGL(k_gather<R>, dim3(nb), dim3(kScanBlock), 0, s, w);
+    const uint32_t shift = tile_shift(w.tile_variant);
+    hipLaunchKernelGGL(k_gather<R>, dim3(nb), dim3(kScanBlock), 0, s, w, shift);
+    if (nb == 1u) return;
     const int from = scan_block_sums(w.blocksum, nb, s);
-    hipLaunchKernelGGL(k_offsets<R>, dim3(nb), dim3(kBlock), 0, s, w, from, tile_shift(w.tile_variant));
+    hipLaunchKernelGGL(k_offsets<R>, dim3(nb), dim3(kBlock), 0, s, w, from, shift);
 }
 
 template <class R>
@@ -4176,7 +4230,7 @@ void launch_step(const WorldView<R>& w0, hipStream_t s, hipEvent_t* marks)
     hipLaunchKernelGGL(k_wall<R>, dim3(gwall + gins), dim3(kBlock), 0, s, w, gwall);
     if (w.nwf > 0) {
         const uint32_t nw1 = (uint32_t)w.nwf + 1u;
-        scan_u32(w.wcnt, nw1, w.woff, w.blocksum, nullptr, s);
+        if (w.nwf > kWallScanFaces) scan_u32(w.wcnt, nw1, w.woff, w.blocksum, nullptr, s);
         hipLaunchKernelGGL(k_wall_bucket<R>, dim3(grid_for(w.ev_cap, 1024)), dim3(kBlock), 0, s, w);
         if (w.nwf <= kWallWaveFaces)
             hipLaunchKernelGGL((k_wall_reduce<R, 64>), dim3(grid_for((uint64_t)w.nwf * 64)), dim3(kBlock), 0, s, w);

@@ -1079,12 +1079,12 @@ int World::step(int n)
                 kn_due = 1;
                 kn_passes = std::max(kn_passes, c.smoothing_passes);
             }
-        // the tuner times each cell-tile configuration on one of the first
-        // kTileVariants steps, with or without step timing
+        // the tuner times each cell-tile configuration on two of the first
+        // kTuneSteps steps, with or without step timing
         // and, as the flow develops, it times the conservation kernel's two
         // occupancies on the collide phase of the last kConsVariants steps of
         // every kConsRetune (not on decomposition steps)
-        const bool tile_tuning = autotune && tune_step < kTileVariants;
+        const bool tile_tuning = autotune && tune_step < kTuneSteps;
         const uint64_t phase = steps_done % kConsRetune;
         const bool cons_tuning = autotune && !tile_tuning && !kn_due && precision == UGX_FP32_STATE && has_bgk
                                  && !has_macro && phase >= kConsRetune - kConsVariants;
@@ -1098,7 +1098,7 @@ int World::step(int n)
                 }
                 marks = tune_ev.data();
             }
-            if (tile_tuning) variant = tune_step;
+            if (tile_tuning) variant = tune_step % kTileVariants;
             if (cons_tuning) cvariant = (int)(phase - (kConsRetune - kConsVariants));
         }
         const bool graph = use_graphs && !marks && !kn_due;
@@ -1134,8 +1134,8 @@ int World::step(int n)
             float ms = 0.0f;
             if (tile_tuning) {
                 HIP_TRY(hipEventElapsedTime(&ms, marks[6], marks[7]));
-                tune_ms[variant] += ms;
-                if (++tune_step == kTileVariants) {
+                tune_ms[variant] = (tune_step < kTileVariants) ? (double)ms : std::min(tune_ms[variant], (double)ms);
+                if (++tune_step == kTuneSteps) {
                     int best = 0;
                     for (int v = 1; v < kTileVariants; ++v) if (tune_ms[v] < tune_ms[best]) best = v;
                     tile_variant = best;

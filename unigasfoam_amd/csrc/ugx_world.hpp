@@ -221,8 +221,12 @@ struct World {
     // HIP-graph replay of whole steps: one executable graph per buffer parity
     // (the step's kernels and arguments are otherwise fixed for a world)
     bool use_graphs = false;
-    // autotuner: each of the first kTileVariants steps times one cell-tile
-    // configuration on the live case (results do not depend on it)
+    // autotuner: each of the first kTuneSteps steps times one cell-tile
+    // configuration on the live case (results do not depend on it), every
+    // configuration twice, the faster time counting: the first launch of a kernel
+    // is slow and irregular (channel of 1e5, FP32: timed once, a configuration
+    // of 36 us was taken where another ran in 21)
+    static constexpr int kTuneSteps = 2 * kTileVariants;
     bool autotune = true;
     int tile_variant = 0;
     uint32_t move_grid = 0;       // resident blocks of the move kernel
