@@ -154,8 +154,8 @@ struct WorldView {
     const double* cw;         // [nc]
     int32_t has_weighting;
     uint32_t* cstart;         // [cap]
-    uint32_t* wclone;         // [cap + 1]
-    uint32_t* wcoff;          // [cap + 1]
+    uint32_t* wclone;         // [cap + 1] clone count of a slot
+    uint32_t* wcoff;          // [cap + 1] per chunk of slots its clones, then the offset of the first
     uint32_t* wbsum;          // scan scratch for cap entries
     // NTC subcells (noTimeCounter.C:97-161): with any cell split, per cell
     // its packed levels (x | y << 8 | z << 16) and the offset of its subcell
