@@ -66,32 +66,14 @@ __device__ inline void wave_run_inc(uint32_t* ctr, const uint32_t (&key)[U], con
     for (int u = 0; u < U; ++u) rank[u] = __shfl(base[u], (int)head[u]) + (lane - head[u]);
 }
 
-// Adds v to counters[ccase][idx]; one atomic per wave when the wave's
-// non-zero contributions share a case.  Called by every lane of the wave.
-__device__ inline void case_add(unsigned long long* counters, int ccase, int idx, unsigned long long v)
-{
-    unsigned long long nz = __ballot(v != 0ull);
-    if (nz == 0ull) return;
-    int leader = __ffsll(nz) - 1;
-    int lc = __shfl(ccase, leader);
-    unsigned long long other = __ballot(v != 0ull && ccase != lc);
-    if (other == 0ull) {
-        unsigned long long s = v;
-        for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
-        if ((int)__lane_id() == leader) atomicAdd(&counters[(size_t)lc * kCntNum + idx], s);
-    } else if (v != 0ull) {
-        atomicAdd(&counters[(size_t)ccase * kCntNum + idx], v);
-    }
-}
-
-
 // Per-thread counters of one case, reduced over the block at kernel end so
 // that a kernel issues one global atomic per counter per block instead of
 // one per wave.  Slots: 0 deleted, 1 wall hits, 2 track errors, 3 inserted.
 // T is the per-thread count type; 32-bit counts go to the global counters
 // before one of them could pass 2^31.
 // Slot maps: M = 0 the tracking counters above, M = 1 the cell weighting's
-// (0 clones, 1 removals).
+// (0 clones, 1 removals), M = 2 the collisions' (0 candidates, 1 collisions,
+// 2 BGK selections).
 template <class T, int M = 0>
 struct TCount {
     int ccase;
@@ -103,7 +85,8 @@ __device__ inline int tcount_idx(int k)
 {
     constexpr int kMap0[4] = {kCntDeleted, kCntWallHits, kCntTrackErrors, kCntInserted};
     constexpr int kMap1[4] = {kCntCloned, kCntWeightDeleted, kCntCloned, kCntCloned};
-    return M == 0 ? kMap0[k] : kMap1[k];
+    constexpr int kMap2[4] = {kCntCandidates, kCntCollisions, kCntBgk, kCntBgk};
+    return M == 0 ? kMap0[k] : M == 1 ? kMap1[k] : kMap2[k];
 }
 
 template <int M>
@@ -186,6 +169,18 @@ __device__ inline void tcount_block_flush(const TCount<T, M>& t, unsigned long l
     }
 }
 
+// Where the blocks of a step's kernels add their counts: a case's counters, or,
+// in a world of one case, one of kCntSlots copies of them, which k_end_step
+// folds in.  Atomics on one address take 6 to 8 ns each here, one after the
+// other: with an atomic per wave and counter k_collide of the mixed nozzle
+// (8.4e5 cells) was 388 us, with one per block and copy 235 (the selections'
+// reservation, one more per wave, went too); k_weight of the expansion 92, 71.
+template <class R>
+__device__ inline unsigned long long* step_counters(const WorldView<R>& w)
+{
+    return (w.ncases == 1) ? w.cslots + (blockIdx.x % kCntSlots) * kCntStride : w.counters;
+}
+
 __device__ inline uint32_t wave_incl_scan_u32(uint32_t v)
 {
     const int lane = (int)__lane_id();
@@ -258,7 +253,7 @@ __global__ void __launch_bounds__(kBeginBlock) k_begin_step(WorldView<R> w)
         if (cs.active && cs.coll_model == UGX_COLL_HYBRID) cs.kn_time += cs.dt;
     }
     if (tid == 0u) {
-        w.st->n_ins = 0u; w.st->nwall = 0u; w.st->nsel = 0u;
+        w.st->n_ins = 0u; w.st->nwall = 0u;
         w.st->nev_peak = max(w.st->nev_peak, w.st->nev);
         w.st->nev = 0u;
     }
@@ -927,7 +922,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof
         const uint64_t ob = base0 + (uint64_t)oldest * cstride;
         move_flush(w, stage, wv, oldest, ob, chunk_valid(ob, n0), lane);
     }
-    tcount_block_flush(tc, w.counters);
+    tcount_block_flush(tc, step_counters(w));
 }
 
 // Diffuse-wall continuation of the queued tracks, as block `block` of `nblocks`.
@@ -982,7 +977,7 @@ __global__ void __launch_bounds__(kBlock) k_wall(WorldView<R> w, uint32_t nwb)
     TCount<unsigned long long> tc{-1, {0ull, 0ull, 0ull, 0ull}};
     if (walls) wall_body(w, block, nwb, tc);
     else inflow_body(w, block, gridDim.x - nwb, tc);
-    tcount_block_flush(tc, w.counters);
+    tcount_block_flush(tc, step_counters(w));
 }
 
 // ---------------------------------------------------------- cell weighting
@@ -1089,7 +1084,7 @@ __global__ void __launch_bounds__(kBlock) k_weight(WorldView<R> w)
         tcount_add(tc, w.counters, ccase, 1, del ? 1u : 0u);
         return k;
     });
-    tcount_block_flush(tc, w.counters);
+    tcount_block_flush(tc, step_counters(w));
 }
 
 // The clones: copies of a slot, in slot order, from n_all on.  Nothing is
@@ -2971,29 +2966,17 @@ __device__ inline void bgk_select(const WorldView<R>& w, const CaseDev& cs, uint
     }
 }
 
-// Exclusive wave prefix of v and one atomic reservation per wave on *ctr;
-// called by all 64 lanes.  Returns the lane's base.
-__device__ inline uint32_t wave_reserve(uint32_t* ctr, uint32_t v)
-{
-    const uint32_t lane = __lane_id();
-    uint32_t incl = v;
-    for (int o = 1; o < 64; o <<= 1) {
-        const uint32_t u = __shfl_up(incl, o);
-        if ((int)lane >= o) incl += u;
-    }
-    const uint32_t total = __shfl(incl, 63);
-    uint32_t base = 0;
-    if (lane == 63u && total) base = atomicAdd(ctr, total);
-    base = __shfl(base, 63);
-    return base + incl - v;
-}
-
-// Lane per cell: BGK-family parameters and selections, NTC collisions.
+// Lane per cell: BGK-family parameters and selections, NTC collisions.  Every
+// 2^spread-th lane has a cell.  A wave takes as long as its longest cell and
+// runs every branch that one of its cells takes, so in a world of too few
+// cells to fill the chip with full waves the cells are spread over more waves
+// (collide_spread).
 template <class R>
-__global__ void __launch_bounds__(kBlock) k_collide(WorldView<R> w)
+__global__ void __launch_bounds__(kBlock) k_collide(WorldView<R> w, uint32_t spread)
 {
-    const uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;
-    const bool on = c < (uint32_t)w.nc;
+    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t c = t >> spread;
+    const bool on = c < (uint32_t)w.nc && (t & ((1u << spread) - 1u)) == 0u;
     unsigned long long cand = 0ull, coll = 0ull;
     uint32_t nrel = 0u, b = 0u, nC = 0u;
     int ccase = 0;
@@ -3025,17 +3008,15 @@ __global__ void __launch_bounds__(kBlock) k_collide(WorldView<R> w)
         w.bgkp[c] = P;
         w.raise[c] = 0ull;
     }
-    const uint32_t base = wave_reserve(&w.st->nsel, nrel);
     if (bgk) {
-        w.bgkp[c].sel_base = base;
+        w.bgkp[c].sel_base = b;
         w.bgkp[c].nrel = nrel;
     }
     __shared__ uint16_t s_perm[kSelLds * kBlock];
-    if (nrel) bgk_select<R>(w, w.cases[ccase], c, b, nC, nrel, base, A, &s_perm[threadIdx.x]);
+    if (nrel) bgk_select<R>(w, w.cases[ccase], c, b, nC, nrel, b, A, &s_perm[threadIdx.x]);
     if (dsmc && nC >= 2u) ntc_cell<R>(w, w.cases[ccase], c, b, nC, A, cand, coll);
-    case_add(w.counters, ccase, kCntCandidates, cand);
-    case_add(w.counters, ccase, kCntCollisions, coll);
-    case_add(w.counters, ccase, kCntBgk, (unsigned long long)nrel);
+    const TCount<unsigned long long, 2> tc{on ? ccase : -1, {cand, coll, (unsigned long long)nrel, 0ull}};
+    tcount_block_flush(tc, step_counters(w));
 }
 
 // interpolationCellPoint at position x (cell frame) of cell c: the tet of
@@ -3327,14 +3308,13 @@ template <class R, bool Macro, int kConsReg>
 __device__ __attribute__((always_inline)) inline void bgk_conserve_body(const WorldView<R>& w)
 {
     const uint32_t tid = threadIdx.x;
-    const uint32_t lane = tid & 63u, g = lane >> 3, j = lane & 7u;
+    const uint32_t lane = tid & 63u, j = lane & 7u;
     const uint32_t c = (blockIdx.x * blockDim.x + tid) >> 3;
     bool perform = false, usp = false;
     uint32_t b = 0, e = 0, sb = 0, nrel = 0;
     int ccase = 0;
     double T = 0.0, U0 = 0.0, U1 = 0.0, U2 = 0.0, M = 0.0, N = 0.0;
     int one_sp = -1;   // the global species of a single-species case, else -1
-    (void)g;
     if (c < (uint32_t)w.nc) {
         // the cell's own rows are loaded along with its case, not after it
         const uint32_t cb = w.off[c], ce = w.off[c + 1];
@@ -3994,6 +3974,18 @@ __global__ void k_end_step(WorldView<R> w)
         }
     }
     if (c == 0) w.st->n = w.st->n_new;
+    // the copies of a single case's counters (the two above are not among them)
+    if (w.ncases == 1 && c < kCntNum) {
+        unsigned long long v[kCntSlots], sum = 0ull;
+#pragma unroll
+        for (int q = 0; q < kCntSlots; ++q) v[q] = w.cslots[q * kCntStride + c];
+#pragma unroll
+        for (int q = 0; q < kCntSlots; ++q) sum += v[q];
+        if (sum != 0ull) {
+            w.counters[c] += sum;
+            for (int q = 0; q < kCntSlots; ++q) w.cslots[q * kCntStride + c] = 0ull;
+        }
+    }
 }
 
 template <class R>
@@ -4122,6 +4114,22 @@ static inline unsigned grid_for(uint64_t n, unsigned cap_blocks = 8192)
 static inline unsigned count_grid(uint64_t cap)
 {
     return grid_for((cap + kCountUnroll - 1) / kCountUnroll);
+}
+
+// Lanes per cell of k_collide as a power of two: the cells of a small world are
+// spread over up to kCollideWaves waves, those of dense cells (kDenseCell slots
+// and more per cell) over as many as are resident (channel of 500 cells of 200:
+// 33 us, 22; FP64 cylinder of 5141 of 150: 73, 50; cylinder of 8e4 of 625: 477,
+// 402).  Cells of 40 gain nothing past one wave per SIMD and lose memory
+// coalescing (DSMC nozzle of 5.9e4 cells: 92 us, spread over 1832 waves 102).
+constexpr uint64_t kCollideWaves = 1536, kCollideWavesDense = 3072, kDenseCell = 128;
+
+static inline uint32_t collide_spread(uint32_t nc, uint64_t cap)
+{
+    const uint64_t most = (cap >= kDenseCell * nc) ? kCollideWavesDense : kCollideWaves;
+    uint32_t k = 0u;
+    while (k < 6u && ((uint64_t)nc << (k + 1u)) / 64u <= most) ++k;
+    return k;
 }
 
 // Blocks of the weighting passes (they stride over the chunks).
@@ -4322,8 +4330,9 @@ void launch_step(const WorldView<R>& w0, hipStream_t s, hipEvent_t* marks)
     launch_tiles<R>(w, s, false);
     mark(7);
     if (w.has_collide) {
-        const unsigned gcell = (unsigned)(((uint64_t)w.nc + kBlock - 1) / kBlock);
-        hipLaunchKernelGGL(k_collide<R>, dim3(gcell), dim3(kBlock), 0, s, w);
+        const uint32_t spread = collide_spread((uint32_t)w.nc, w.cap);
+        const unsigned gcell = (unsigned)((((uint64_t)w.nc << spread) + kBlock - 1) / kBlock);
+        hipLaunchKernelGGL(k_collide<R>, dim3(gcell), dim3(kBlock), 0, s, w, spread);
         if (w.has_macro)
             hipLaunchKernelGGL(k_point_fields<R>, dim3(grid_for(w.npts)), dim3(kBlock), 0, s, w);
         if (w.has_bgk) {

@@ -15,7 +15,6 @@ struct DevState {
     uint32_t big_tiles;     // cell tiles handled by the global-memory path
     uint32_t nwall;         // queued diffuse-wall tracks this step
     uint32_t ntiles;        // cell tiles of this step's sort
-    uint32_t nsel;          // BGK selections this step
     uint32_t nev;           // wall-hit events this step
     uint32_t nev_peak;      // largest nev of a finished step
     uint32_t evover;        // a step had more wall hits than the event buffer holds
@@ -62,6 +61,12 @@ enum CounterIdx {
     kCntWallHits, kCntTrackErrors, kCntSampled, kCntParticleSteps, kCntCloned, kCntWeightDeleted, kCntNum
 };
 
+// Copies of the counters that a step's kernels add to (step_counters), each on
+// a line of its own.
+constexpr int kCntSlots = 32;
+constexpr int kCntStride = 16;
+static_assert(kCntNum <= kCntStride, "counter slots");
+
 template <class R>
 struct WorldView {
     Parts<R> a;               // current particle buffers
@@ -104,7 +109,7 @@ struct WorldView {
     double* mom;              // [nc][kNMom] per-cell sums for the BGK family
     BgkP* bgkp;               // [nc]
     unsigned long long* raise;// [nc] USP maxProb raise (bits of a positive double)
-    uint32_t* sel_slot;       // [cap] BGK selections: sorted slot of each (cell-major, in selection order)
+    uint32_t* sel_slot;       // [cap] BGK selections: sorted slot of each (a cell's from its first slot on)
     int32_t ns_max;           // largest species count of a case
     int32_t sum_level;        // largest sampler level of a case (0, 1, 2)
     int32_t has_collide;      // some case collides (DSMC or BGK family)
@@ -125,6 +130,7 @@ struct WorldView {
     int32_t has_bgk;          // some case runs a BGK-family model
     uint32_t* blocksum;       // scan scratch
     unsigned long long* counters; // [ncases*kCntNum]
+    unsigned long long* cslots;   // [kCntSlots*kCntStride] copies of a single case's counters, 0 between steps
     DevState* st;
     int32_t nc;
     uint32_t cap;

@@ -360,7 +360,7 @@ void World::release()
                      (void**)&d_tile_first, (void**)&d_tile_p0, (void**)&d_tile_case,
                      (void**)&d_mom, (void**)&d_bgkp, (void**)&d_raise,
                      (void**)&d_sel_slot,
-                     (void**)&d_blocksum, (void**)&d_counters, (void**)&d_st,
+                     (void**)&d_blocksum, (void**)&d_counters, (void**)&d_cslots, (void**)&d_st,
                      (void**)&d_wq_slot, (void**)&d_wq_info, (void**)&d_wq_tau,
                      (void**)&d_wface, (void**)&d_wgeo, (void**)&d_wcell, (void**)&d_ev, (void**)&d_ev_key,
                      (void**)&d_wcnt, (void**)&d_woff, (void**)&d_bkey, (void**)&d_bidx, (void**)&d_wsamp,
@@ -565,6 +565,7 @@ WorldView<R> World::view() const
     w.has_bgk = has_bgk;
     w.blocksum = d_blocksum;
     w.counters = d_counters;
+    w.cslots = d_cslots;
     w.st = d_st;
     w.nc = nc;
     w.cap = cap;
@@ -940,6 +941,8 @@ int World::build(std::vector<CaseSpec>& specs, int prec, int device, uint64_t ca
     if ((rc = dalloc(d_blocksum, nbs))) return rc;
     std::vector<unsigned long long> zcnt(specs.size() * kCntNum, 0ull);
     if ((rc = up(d_counters, zcnt))) return rc;
+    std::vector<unsigned long long> zslots((size_t)kCntSlots * kCntStride, 0ull);
+    if ((rc = up(d_cslots, zslots))) return rc;
     DevState st{};
     std::vector<DevState> vst(1, st);
     if ((rc = up(d_st, vst))) return rc;

@@ -134,6 +134,7 @@ struct World {
     int32_t ns_max = 1, sum_level = 0, has_collide = 0, has_bgk = 0;
     uint32_t* d_blocksum = nullptr;
     unsigned long long* d_counters = nullptr;
+    unsigned long long* d_cslots = nullptr;
     DevState* d_st = nullptr;
     uint32_t* d_wq_slot = nullptr;
     uint32_t* d_wq_info = nullptr;
