@@ -1392,6 +1392,8 @@ constexpr uint32_t kMaxTileCells = 512u / kCellW + 2u;   // cells of the largest
 constexpr int kCountTiles = 4;                           // tiles per block of k_count_tiles
 // Largest grid of the occupancy count (blocks stride over the step's tile groups).
 constexpr uint64_t kCountGrid = 8192;
+// Tile tables up to this length get a block per tile.
+constexpr uint64_t kCountSmall = 8192;
 
 // Class-7 counting of the slots [begin, n + n_ins) as block `block` of
 // `nblocks`: the inflow and clones of a step, or every slot for the sort
@@ -1429,7 +1431,7 @@ __global__ void k_count(WorldView<R> w)
 }
 
 // Classes of the simulators that were in the cells of TPB consecutive tiles of
-// the previous sort (one block per TPB tiles), in windows of kCountWindow
+// the previous sort (one block per tpb <= TPB tiles), in windows of kCountWindow
 // slots.  The rank within (old cell, class) follows the order of the slots:
 // within each 64-slot chunk of the window, ballots per class give a
 // simulator's rank among the same cell's and class's earlier slots of the
@@ -1441,7 +1443,7 @@ __global__ void k_count(WorldView<R> w)
 constexpr uint32_t kCountWindow = 512;
 
 template <class R, int Block, int TPB>
-__global__ void __launch_bounds__(Block) __attribute__((amdgpu_waves_per_eu(7))) k_count_tiles(WorldView<R> w, uint32_t ntb)
+__global__ void __launch_bounds__(Block) __attribute__((amdgpu_waves_per_eu(7))) k_count_tiles(WorldView<R> w, uint32_t ntb, uint32_t tpb)
 {
     constexpr int U = kCountWindow / Block;
     constexpr uint32_t kChunks = kCountWindow / 64;
@@ -1463,8 +1465,8 @@ __global__ void __launch_bounds__(Block) __attribute__((amdgpu_waves_per_eu(7)))
     const unsigned long long below = (1ull << lane) - 1ull;
     // the grid is sized for the largest tile table; blocks stride over the
     // groups of this step's tiles
-    for (uint32_t t0 = blockIdx.x * (uint32_t)TPB; t0 < ntiles; t0 += ntb * (uint32_t)TPB) {
-    const uint32_t t1 = min(t0 + (uint32_t)TPB, ntiles);
+    for (uint32_t t0 = blockIdx.x * tpb; t0 < ntiles; t0 += ntb * tpb) {
+    const uint32_t t1 = min(t0 + tpb, ntiles);
     const uint32_t c0 = w.tile_first[t0];
     const uint32_t nct = w.tile_first[t1] - c0;
     const uint32_t p0 = w.tile_p0[t0];
@@ -4318,11 +4320,14 @@ void launch_step(const WorldView<R>& w0, hipStream_t s, hipEvent_t* marks)
     mark(4);
     // the slots past the existing simulators (a step's clones are few: their
     // blocks are not sized for the bound) are counted beside the tiles
-    const unsigned gct = (unsigned)std::min<uint64_t>(
-        (max_tiles(w.cap, (uint64_t)w.nc) + kCountTiles - 1) / kCountTiles, kCountGrid);
+    // small worlds: a tile per block, so that the tiles' windows run side by side
+    // (channels of 1e5: 22 to 24 us, 9 to 11; four per block in larger ones)
+    const uint64_t nt = max_tiles(w.cap, (uint64_t)w.nc);
+    const uint32_t tpb = (nt <= kCountSmall) ? 1u : (uint32_t)kCountTiles;
+    const unsigned gct = (unsigned)std::min<uint64_t>((nt + tpb - 1) / tpb, kCountGrid);
     const unsigned gcn = w.has_weighting ? 512u
                          : w.n_inflow > 0 ? grid_for(((uint64_t)w.max_ins + kCountUnroll - 1) / kCountUnroll, 512u) : 0u;
-    hipLaunchKernelGGL((k_count_tiles<R, 256, kCountTiles>), dim3(gct + gcn), dim3(256), 0, s, w, gct);
+    hipLaunchKernelGGL((k_count_tiles<R, 256, kCountTiles>), dim3(gct + gcn), dim3(256), 0, s, w, gct, tpb);
     launch_offsets<R>(w, s);
     mark(5);
     hipLaunchKernelGGL(k_scatter<R>, dim3(count_grid(w.cap)), dim3(kBlock), 0, s, w);
