@@ -1,6 +1,8 @@
 """Passes that change form with the size: offsets beside the populations up to
 1023 cells, wall offsets inside the bucketing up to 4096 faces, and clone
-counts by chunks of 1024 slots.  All equal the oracle, bit for bit."""
+counts by chunks of 1024 slots; and the occupancy count with one or four tiles
+per block, by the length of the tile table.  All equal the oracle, bit for
+bit."""
 import numpy as np
 import pytest
 
@@ -41,3 +43,9 @@ def test_wall_faces_of_one_scan(require_gpu, n):
 @pytest.mark.parametrize("npps", [3, 32, 33, 1500])   # about 100, 1024 and 48000 slots in 32 cells
 def test_clones_by_chunks(require_gpu, npps):
     compare(graded_box(npps=npps), dict(number_density={"Ar": 1.0e20}, T=300.0), 6, 1 << 18)
+
+
+@pytest.mark.parametrize("capacity", [1 << 14, 1 << 20, 1 << 22])   # tables of about 200, 8300 and 33000 tiles
+def test_tiles_of_a_count_block(require_gpu, capacity):
+    spec, fill = workloads.heat_bath(n_cells=9, per_cell=12, side=9.0e-3)
+    compare(spec, fill, 6, capacity)
