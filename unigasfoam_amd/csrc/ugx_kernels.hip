@@ -2128,38 +2128,33 @@ __device__ inline bool samples_now(const TileCase& cs)
     return cs.active && ((cs.step + 1u) % (uint32_t)cs.sample_interval) == 0u;
 }
 
-// What the sums of a cell are needed for.
-struct SumUse {
-    bool sample, hybrid, bgk, adapt;
-    __device__ bool any() const { return sample || hybrid || bgk || adapt; }
-};
-
-__device__ inline SumUse sum_use(const TileCase& cs)
+// What the sums of a cell are needed for; false when for nothing.
+__device__ inline bool sum_use(const TileCase& cs, bool& sample, bool& hybrid, bool& bgk, bool& adapt)
 {
-    SumUse u{false, false, false, false};
-    if (cs.active) {
-        u.sample = ((cs.step + 1u) % (uint32_t)cs.sample_interval) == 0u;
-        u.hybrid = cs.coll_model == UGX_COLL_HYBRID;
-        u.bgk = (cs.coll_model == UGX_COLL_BGK || u.hybrid) && cs.bgk_model != UGX_BGK_NONE;
-        u.adapt = cs.adaptive != 0;
-    }
-    return u;
+    if (!cs.active) return false;
+    sample = ((cs.step + 1u) % (uint32_t)cs.sample_interval) == 0u;
+    hybrid = cs.coll_model == UGX_COLL_HYBRID;
+    bgk = (cs.coll_model == UGX_COLL_BGK || hybrid) && cs.bgk_model != UGX_BGK_NONE;
+    adapt = cs.adaptive != 0;
+    return sample || hybrid || bgk || adapt;
 }
 
 // The totals S of cell c into the sampler, the time sums and the BGK moments;
 // every lane of the cell's group holds the totals and lane j stores its rows.
 // have: pre holds the cell's sampler rows.
 template <int L, int NS, class R>
-__device__ __attribute__((always_inline)) inline void store_sums(const WorldView<R>& w, uint32_t c, uint32_t j, const TileCase& cs, const SumUse& use,
-                                  const double (&S)[SumRows<L, NS>::kN], const SampPre& pre, bool have)
+__device__ __attribute__((always_inline)) inline void store_sums(const WorldView<R>& w, uint32_t c, uint32_t j,
+                                                                 double dt, int ns, bool full, bool sample,
+                                                                 bool hybrid, bool bgk, bool adapt,
+                                                                 const double (&S)[SumRows<L, NS>::kN],
+                                                                 const SampPre& pre, bool have)
 {
     constexpr bool MS = NS > 1;
     constexpr int B = SumRows<L, NS>::kBase;
-    const double dt = cs.dt;
-    if (use.sample) {
+    if (sample) {
         int rows[5];
         double v[5];
-        samp_lane_rows<L, NS>(j, cs.ns, cs.sampler_full != 0, rows);
+        samp_lane_rows<L, NS>(j, ns, full, rows);
         samp_lane_values<L, NS>(j, S, v);
         double* sc = &w.samp[(size_t)c * kNSamp];
 #pragma unroll
@@ -2177,19 +2172,19 @@ __device__ __attribute__((always_inline)) inline void store_sums(const WorldView
     } else {
         vsp = (j == 0u) ? S[UGX_S_N] : 0.0;
     }
-    if (use.hybrid) {
+    if (hybrid) {
         double* ka = &w.knacc[(size_t)kKnRows * c];
         ka[j] += dt * v[0];
         if (MS || j == 0u) ka[8 + j] += dt * vsp;
     }
-    if (use.adapt) {
+    if (adapt) {
         // uniGasDynamicAdapter::adapt (uniGasDynamicAdapter.C:526-547): the
         // cell measurements of every step, weighted by the time step
         double* aa = &w.adacc[(size_t)kKnRows * c];
         aa[j] += dt * v[0];
         if (MS || j == 0u) aa[8 + j] += dt * vsp;
     }
-    if (use.bgk) {
+    if (bgk) {
         double* mo = &w.mom[(size_t)c * kNMom];
 #pragma unroll
         for (int i = 0; i < 3; ++i) {
@@ -2211,23 +2206,37 @@ __device__ inline void tile_sums(const WorldView<R>& w, uint32_t c0, uint32_t nc
     for (uint32_t kb = 0; kb < nct; kb += (Block / 64) * 8) {
         const uint32_t k = kb + wv * 8u + g;
         uint32_t b = 0, e = 0;
-        SumUse use{false, false, false, false};
+        // as in sum_use, but with the time step beside the flags: through sum_use the
+        // loads of the sums below are put one after the other for want of registers
+        // (cell sums of two species, level 2, 1500 per cell, FP32: 450 us, like this
+        // 321; with flags kept in a struct k_tile of two species also lost a wave per
+        // SIMD: cylinder of 5e7 by tiles 4150 us, 3430)
+        bool sample = false, hybrid = false, bgk = false, adapt = false;
+        double dt = 0.0;
         const uint32_t c = c0 + k;
         TileCase cs{};
         if (k < nct) {
             const int ci = s_cc[k];
             cs = (ci == case0) ? *s_tc : tile_case_of(w.cases[ci]);
-            use = sum_use(cs);
-            if (use.any()) { b = s_off[k]; e = s_off[k + 1]; }
+            if (cs.active) {
+                sample = ((cs.step + 1u) % (uint32_t)cs.sample_interval) == 0u;
+                hybrid = cs.coll_model == UGX_COLL_HYBRID;
+                bgk = (cs.coll_model == UGX_COLL_BGK || hybrid) && cs.bgk_model != UGX_BGK_NONE;
+                adapt = cs.adaptive != 0;
+                if (sample || hybrid || bgk || adapt) { b = s_off[k]; e = s_off[k + 1]; }
+                dt = cs.dt;
+            }
         }
-        if (__ballot(use.any()) == 0ull) continue;
+        const bool need = sample || hybrid || bgk || adapt;
+        if (__ballot(need) == 0ull) continue;
         double S[NR];
 #pragma unroll
         for (int q = 0; q < NR; ++q) S[q] = 0.0;
         cell_partials<L, NS, R, Acc>(w, A, b + j, e, S);
 #pragma unroll
         for (int q = 0; q < NR; ++q) S[q] = group8_total(S[q]);
-        store_sums<L, NS, R>(w, c, j, cs, use, S, pre, pre.valid && kb == 0u);
+        store_sums<L, NS, R>(w, c, j, dt, cs.ns, cs.sampler_full != 0, need && sample, need && hybrid, need && bgk,
+                             need && adapt, S, pre, pre.valid && kb == 0u);
     }
 }
 
@@ -2556,10 +2565,10 @@ __global__ void __launch_bounds__(kBlock) k_cell_sums(WorldView<R> w)
     __syncthreads();
     TileCase cs = s_tc;
     if (ci != case0) cs = tile_case_of(w.cases[ci]);
-    SumUse use{false, false, false, false};
-    if (c < nc) use = sum_use(cs);
-    if (!use.any()) e = b;
-    if (__ballot(use.any()) == 0ull) return;
+    bool sample = false, hybrid = false, bgk = false, adapt = false;
+    const bool on = c < nc && sum_use(cs, sample, hybrid, bgk, adapt);
+    if (!on) e = b;
+    if (__ballot(on) == 0ull) return;
     // a single-species case: its species' constants
     const double m1 = (NS > 1) ? 0.0 : w.sp.mass[cs.sp_base];
     const double rd1 = (NS > 1) ? 0.0 : (double)w.sp.rotdof[cs.sp_base];
@@ -2594,7 +2603,8 @@ __global__ void __launch_bounds__(kBlock) k_cell_sums(WorldView<R> w)
     for (; i < e; i += 8u) pass(i, std::integral_constant<int, 1>{});
 #pragma unroll
     for (int q = 0; q < NR; ++q) S[q] = group8_total(S[q]);
-    store_sums<L, NS, R>(w, c, j, cs, use, S, SampPre{{0.0, 0.0, 0.0, 0.0, 0.0}, false}, false);
+    store_sums<L, NS, R>(w, c, j, cs.dt, cs.ns, cs.sampler_full != 0, sample, hybrid, bgk, adapt, S,
+                         SampPre{{0.0, 0.0, 0.0, 0.0, 0.0}, false}, false);
 }
 
 // ------------------------------------------------------------- collisions
