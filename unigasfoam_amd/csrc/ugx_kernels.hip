@@ -66,6 +66,37 @@ __device__ inline void wave_run_inc(uint32_t* ctr, const uint32_t (&key)[U], con
     for (int u = 0; u < U; ++u) rank[u] = __shfl(base[u], (int)head[u]) + (lane - head[u]);
 }
 
+// The same with one atomic per distinct key of the wave and key set, found by a
+// ballot per key: for keys that repeat but not in runs, on counters that many
+// waves add to at the same time, because atomics on one counter take turns
+// (count_shared).  Called by every lane of the wave.
+template <int U>
+__device__ inline void wave_key_inc(uint32_t* ctr, const uint32_t (&key)[U], const bool (&active)[U],
+                                    uint32_t (&rank)[U])
+{
+    const unsigned lane = __lane_id();
+    uint32_t base[U], head[U], place[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        base[u] = 0u;
+        head[u] = 0u;
+        place[u] = 0u;
+        for (unsigned long long todo = __ballot(active[u]); todo != 0ull;) {
+            const int leader = __ffsll(todo) - 1;
+            const uint32_t lkey = __shfl(key[u], leader);
+            const unsigned long long same = __ballot(key[u] == lkey) & todo;
+            if ((int)lane == leader) base[u] = atomicAdd(&ctr[lkey], (uint32_t)__popcll(same));
+            if ((same >> lane) & 1ull) {
+                head[u] = (uint32_t)leader;
+                place[u] = (uint32_t)__popcll(same & ((1ull << lane) - 1ull));
+            }
+            todo &= ~same;
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) rank[u] = __shfl(base[u], (int)head[u]) + place[u];
+}
+
 // Per-thread counters of one case, reduced over the block at kernel end so
 // that a kernel issues one global atomic per counter per block instead of
 // one per wave.  Slots: 0 deleted, 1 wall hits, 2 track errors, 3 inserted.
@@ -1443,7 +1474,7 @@ __global__ void k_count(WorldView<R> w)
 constexpr uint32_t kCountWindow = 512;
 
 template <class R, int Block, int TPB>
-__global__ void __launch_bounds__(Block) __attribute__((amdgpu_waves_per_eu(7))) k_count_tiles(WorldView<R> w, uint32_t ntb, uint32_t tpb)
+__global__ void __launch_bounds__(Block) __attribute__((amdgpu_waves_per_eu(7))) k_count_tiles(WorldView<R> w, uint32_t ntb, uint32_t tpb, bool shared)
 {
     constexpr int U = kCountWindow / Block;
     constexpr uint32_t kChunks = kCountWindow / 64;
@@ -1513,7 +1544,8 @@ __global__ void __launch_bounds__(Block) __attribute__((amdgpu_waves_per_eu(7)))
             }
             other[u] = d[u] != kDead && cls[u] == kClassOther;
         }
-        wave_run_inc<U>(w.ocnt, d, other, ro);
+        if (shared) wave_key_inc<U>(w.ocnt, d, other, ro);
+        else wave_run_inc<U>(w.ocnt, d, other, ro);
         // ranks within the chunk (entries u * Block + tid: chunk u * Block / 64 + wave)
 #pragma unroll
         for (int u = 0; u < U; ++u) {
@@ -4128,6 +4160,15 @@ static inline unsigned count_grid(uint64_t cap)
     return grid_for((cap + kCountUnroll - 1) / kCountUnroll);
 }
 
+// Whether the occupancy count shares an atomic between a wave's equal keys: where
+// the simulators that crossed several cells meet on few counters, that is with
+// many slots per cell (whole scan phase; runs / shared.  Channels of 1000 cells:
+// of 1e4 simulators, one cell crossed per step 245 / 195 us, ten 497 / 288; of
+// 1000, 52 / 45 and 77 / 68.  Cylinder of 625 per cell 571 / 546.  Boxes of 400
+// per cell 69 / 84, of 30 per cell 40 / 76.)
+constexpr uint64_t kCountShared = 768;
+static inline bool count_shared(uint32_t nc, uint64_t cap) { return cap >= kCountShared * nc; }
+
 // Lanes per cell of k_collide as a power of two: the cells of a small world are
 // spread over up to kCollideWaves waves, those of dense cells (kDenseCell slots
 // and more per cell) over as many as are resident (channel of 500 cells of 200:
@@ -4337,7 +4378,8 @@ void launch_step(const WorldView<R>& w0, hipStream_t s, hipEvent_t* marks)
     const unsigned gct = (unsigned)std::min<uint64_t>((nt + tpb - 1) / tpb, kCountGrid);
     const unsigned gcn = w.has_weighting ? 512u
                          : w.n_inflow > 0 ? grid_for(((uint64_t)w.max_ins + kCountUnroll - 1) / kCountUnroll, 512u) : 0u;
-    hipLaunchKernelGGL((k_count_tiles<R, 256, kCountTiles>), dim3(gct + gcn), dim3(256), 0, s, w, gct, tpb);
+    hipLaunchKernelGGL((k_count_tiles<R, 256, kCountTiles>), dim3(gct + gcn), dim3(256), 0, s, w, gct, tpb,
+                       count_shared((uint32_t)w.nc, w.cap));
     launch_offsets<R>(w, s);
     mark(5);
     hipLaunchKernelGGL(k_scatter<R>, dim3(count_grid(w.cap)), dim3(kBlock), 0, s, w);
