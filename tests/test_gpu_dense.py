@@ -2,10 +2,14 @@
 neighbours in a step: what is done for them must not grow out of proportion.
 The bounds are ratios of times of one run, between those measured with and
 without the forms that keep to them."""
+import numpy as np
 import pytest
 
-from unigasfoam_amd import workloads
+from oracle.orc import OracleCase
+from unigasfoam_amd import abi, workloads
 from unigasfoam_amd.core import Case
+from unigasfoam_amd.mesh import box_mesh
+from unigasfoam_amd.spec import Boundary, CaseSpec
 
 pytestmark = pytest.mark.gpu
 
@@ -32,3 +36,43 @@ def test_count_of_cells_crossed(require_gpu):
     more by atomics on 1000 counters (1.5 times as long, 2.0 with an atomic per
     simulator)."""
     assert phase_us(10000, 5, "scan") < 1.75 * phase_us(10000, 1, "scan")
+
+
+def test_sums_of_many_hits_per_face(require_gpu):
+    """Ten times the hits on the two faces of a channel (570 and 5700 each)."""
+    assert phase_us(1000, 10, "wall") < 20.0 * phase_us(1000, 1, "wall")
+
+
+def same_wall_sums(spec, fill, steps, capacity):
+    """The wall sums after `steps` steps, equal to the oracle's; hits per face."""
+    g = Case(spec, precision="fp64", capacity=capacity)
+    o = OracleCase(spec, capacity=1 << 19)
+    for c in (g, o):
+        c.fill(**fill)
+        c.step(steps)
+    assert np.array_equal(g.wall_samples(), o.wall_samples())
+    hits = g.counters()["wall_hits"] / steps / g.wall_face_count()
+    g.close()
+    o.close()
+    return hits
+
+
+@pytest.mark.parametrize("per_cell, least, most", [(420, 180, 250), (480, 230, 290), (1060, 470, 560),
+                                                   (2100, 950, 1100), (10000, 4500, 5200)])
+def test_order_of_many_hits(require_gpu, per_cell, least, most):
+    """Faces of less and more hits than a wave orders at a time (256), odd and even
+    numbers of stretches, one, two and several merges."""
+    spec, fill = workloads.couette(n_cells=10, per_cell=per_cell, dt=5.0e-7, gas="Ar")
+    spec.boundaries[1].kind = abi.BND_SPECULAR
+    hits = same_wall_sums(spec, fill, 3, 1 << 20)
+    assert least < hits < most, hits
+
+
+def test_order_of_many_hits_on_many_faces(require_gpu):
+    """More than 8192 faces, 16 lanes each, that order 64 hits at a time."""
+    pt = {k: abi.WALL for k in ("xmin", "xmax", "ymin", "ymax", "zmin", "zmax")}
+    mesh = box_mesh((0.0, 0.0, 0.0), (2.1, 1.0e-3, 1.0e-3), (2100, 1, 1), pt)
+    spec = CaseSpec(mesh=mesh, species=[workloads.ARGON, workloads.N2], delta_t=2.0e-5, n_equivalent_particles=1.0e9,
+                    collision_model="none", boundaries=[Boundary(p, abi.BND_SPECULAR) for p in pt])
+    hits = same_wall_sums(spec, dict(number_density={"Ar": 2.0e19, "N2": 2.0e19}, T=300.0), 2, 1 << 23)
+    assert 64 < hits < 256, hits

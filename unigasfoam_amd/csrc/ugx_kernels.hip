@@ -1287,12 +1287,15 @@ __device__ inline void wall_terms(const double U[3], double e, const double n[3]
 // A group of G lanes per wall face: sorts the face's hits by key and adds
 // each species' terms in that order, then deltaT times the sums to the face's
 // time sums (at sample steps).  The order of the additions is fixed, so what
-// runs in parallel is the sort (each hit's place is the number of smaller
-// keys; keys are distinct) and the terms of a chunk of hits, which go to LDS;
-// then lane r adds row r of the chunk, hit after hit.  One thread per face
-// with a heap sort in HBM took 149 us per step for the two faces of a 1-D
-// channel (60 hits each) and 65 us for a box of 3174 faces (8 hits each): a
-// serial chain of dependent memory reads.  Here: 17 and 9 us.
+// runs in parallel is the sort (keys are distinct) and the terms of a chunk of
+// hits, which go to LDS; then lane r adds row r of the chunk, hit after hit.  One
+// thread per face with a heap sort in HBM took 149 us per step for the two faces
+// of a 1-D channel (60 hits each) and 65 us for a box of 3174 faces (8 hits
+// each): a serial chain of dependent memory reads.  Here: 17 and 9 us.  More than
+// kKeys hits are ranked kKeys at a time and the stretches merged: by rank alone
+// the work grows with the square of the hits (wall phase of channels with 570,
+// 28,000 and 114,000 hits per face: by heap sort 2.2, 177 and 790 ms, by rank
+// alone 0.26, 241 and 3850 ms, like this 0.16, 8.9 and 41 ms).
 template <class R, int G>
 __global__ void __launch_bounds__(kBlock) k_wall_reduce(WorldView<R> w)
 {
@@ -1313,43 +1316,89 @@ __global__ void __launch_bounds__(kBlock) k_wall_reduce(WorldView<R> w)
     if (n == 0u) return;
     const CaseDev& cs = w.cases[w.cell_case[w.wcell[f]]];
     if (((cs.step + 1u) % (uint32_t)cs.sample_interval) != 0u) return;
-    // the order: in LDS, or for a face with more hits in the key list, whose
-    // contents the buckets hold (entries b.. of it are this face's to use)
+    // kKeys hits at a time by rank: a hit's place is the number of smaller keys
     const bool small = n <= kKeys;
-    uint32_t* const ord = reinterpret_cast<uint32_t*>(w.ev_key) + b;
     for (uint32_t q0 = 0; q0 < n; q0 += kKeys) {
         unsigned long long mk[4];
-        uint32_t mr[4] = {0u, 0u, 0u, 0u};
+        uint32_t mi[4], mr[4] = {0u, 0u, 0u, 0u};
+        wave_sync();
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
-            const uint32_t q = q0 + j + G * (uint32_t)u;
+            const uint32_t p = j + G * (uint32_t)u, q = q0 + p;
             mk[u] = (q < n) ? w.bkey[b + q] : 0ull;
+            mi[u] = (q < n) ? w.bidx[b + q] : 0u;
+            s_key[gi][p] = mk[u];
         }
-        for (uint32_t p0 = 0; p0 < n; p0 += kKeys) {
-            wave_sync();
+        wave_sync();
+        const uint32_t pn = min(kKeys, n - q0);
+        for (uint32_t p = 0; p < pn; ++p) {
+            const unsigned long long k = s_key[gi][p];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) mr[u] += (k < mk[u]) ? 1u : 0u;
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            if (q0 + j + G * (uint32_t)u >= n) continue;
+            if (small) {
+                s_ord[gi][mr[u]] = mi[u];
+            } else {
+                w.bkey[b + q0 + mr[u]] = mk[u];
+                w.bidx[b + q0 + mr[u]] = mi[u];
+            }
+        }
+    }
+    // a face of more hits: its sorted stretches merged pairwise, from the buckets to
+    // the key list and back (the buckets hold what was in it; entries b.. are this
+    // face's to use), each hit's place being its own number in its stretch plus the
+    // number of smaller keys in the other one
+    bool alt = false;   // the order is in ev_key and ev.order, not in bkey and bidx
+    for (uint32_t run = kKeys; run < n; run *= 2u) {
+        __threadfence_block();
+        wave_sync();
+        const unsigned long long* const ks = (alt ? w.ev_key : w.bkey) + b;
+        unsigned long long* const kd = (alt ? w.bkey : w.ev_key) + b;
+        for (uint32_t q0 = 0; q0 < n; q0 += kKeys) {
+            unsigned long long mk[4];
+            uint32_t lo[4], hi[4], to[4];
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
-                const uint32_t p = p0 + j + G * (uint32_t)u;
-                if (p < n) s_key[gi][j + G * (uint32_t)u] = w.bkey[b + p];
+                const uint32_t q = min(q0 + j + G * (uint32_t)u, n - 1u);
+                const uint32_t first = q & ~(2u * run - 1u), second = min(first + run, n);
+                const bool in2 = (q & run) != 0u;
+                mk[u] = ks[q];
+                lo[u] = in2 ? first : second;
+                hi[u] = in2 ? second : min(second + run, n);
+                to[u] = first + (q - (in2 ? second : first)) - lo[u];
             }
-            wave_sync();
-            const uint32_t pn = min(kKeys, n - p0);
-            for (uint32_t p = 0; p < pn; ++p) {
-                const unsigned long long k = s_key[gi][p];
+            for (uint32_t s = run; s != 0u; s >>= 1) {
+                unsigned long long k[4];
+                uint32_t mid[4];
 #pragma unroll
-                for (int u = 0; u < 4; ++u) mr[u] += (k < mk[u]) ? 1u : 0u;
+                for (int u = 0; u < 4; ++u) {
+                    mid[u] = (lo[u] + hi[u]) >> 1;
+                    k[u] = ks[min(mid[u], n - 1u)];
+                }
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const bool open = lo[u] < hi[u], less = k[u] < mk[u];
+                    lo[u] = (open && less) ? mid[u] + 1u : lo[u];
+                    hi[u] = (open && !less) ? mid[u] : hi[u];
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const uint32_t q = q0 + j + G * (uint32_t)u, d = to[u] + lo[u];
+                if (q >= n) continue;
+                kd[d] = mk[u];
+                if (alt) w.bidx[b + d] = w.ev[b + q].order;
+                else w.ev[b + d].order = w.bidx[b + q];
             }
         }
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const uint32_t q = q0 + j + G * (uint32_t)u;
-            if (q >= n) continue;
-            if (small) s_ord[gi][mr[u]] = w.bidx[b + q];
-            else ord[mr[u]] = w.bidx[b + q];
-        }
+        alt = !alt;
     }
     if (!small) __threadfence_block();
     wave_sync();
+    auto ord = [&](uint32_t p) { return small ? s_ord[gi][p] : alt ? w.ev[b + p].order : w.bidx[b + p]; };
     const double* gq = &w.wgeo[(size_t)f * kWGeo];
     const double nw[3] = {gq[0], gq[1], gq[2]};
     const double fA = gq[3];
@@ -1361,7 +1410,7 @@ __global__ void __launch_bounds__(kBlock) k_wall_reduce(WorldView<R> w)
     for (uint32_t p0 = 0; p0 < n; p0 += kChunk) {
         const uint32_t pn = min(kChunk, n - p0);
         if (j < pn) {
-            const WallEv ev = w.ev[small ? s_ord[gi][p0 + j] : ord[p0 + j]];
+            const WallEv ev = w.ev[ord(p0 + j)];
             const double m = w.sp.mass[ev.sp];
             const int rotdof = w.sp.rotdof[ev.sp];
             double t0[kPair], t1[kPair];

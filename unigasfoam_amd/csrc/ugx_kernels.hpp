@@ -29,7 +29,7 @@ struct WallEv {
     uint32_t wf;
     uint32_t sp;
     uint32_t rank;          // arrival number among the step's hits of the face
-    uint32_t pad;
+    uint32_t order;         // room for the sort of a face with many hits
 };
 // Rows of the wall sums per (face, species): ugx_wall_index.
 constexpr int kWRows = UGX_W_COUNT;
@@ -241,7 +241,7 @@ struct WallSink {
         e.wf = (uint32_t)wf;
         e.sp = sp;
         e.rank = rank;
-        e.pad = 0u;
+        e.order = 0u;
         ev[i] = e;
     }
 };
