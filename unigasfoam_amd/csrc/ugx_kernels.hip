@@ -2550,6 +2550,7 @@ __global__ void __launch_bounds__(kBlock) k_order(WorldView<R> w)
         }
     }
     __threadfence_block();   // (a cell's lanes are in one wave)
+    wave_sync();
     if (oc != 0u && !big)
         for (uint32_t i = lo + j; i < e; i += 8u) w.perm[i] = w.scratch[i];
     // the sorted merge list goes to the destination's cell ids, which the gather
@@ -2565,6 +2566,7 @@ __global__ void __launch_bounds__(kBlock) k_order(WorldView<R> w)
             sorted[r] = slot;
         }
         __threadfence_block();
+        wave_sync();
         for (uint32_t i = l + lane; i < z; i += 64u) {
             const bool in = i < o;
             const uint32_t slot = in ? w.perm[i] : sorted[i];
@@ -2572,6 +2574,7 @@ __global__ void __launch_bounds__(kBlock) k_order(WorldView<R> w)
             w.scratch[i + k] = slot;
         }
         __threadfence_block();
+        wave_sync();
         for (uint32_t i = l + lane; i < z; i += 64u) w.perm[i] = w.scratch[i];
     }
 }
