@@ -493,6 +493,10 @@ int ugx_timing_get(ugx_case* c, double* ms_total, int n_phases, int64_t* steps);
  * the fastest; results never depend on it. */
 int ugx_tile_config(ugx_case* c, int32_t* variant, int32_t* threads, int32_t* window, int32_t* lds_simulators,
                     int32_t* tuned);
+/* Runs configuration `variant` (0 to 3) from the next step on instead of the
+ * tuner's choice; -1 has the tuner choose again.  For tests and comparisons of
+ * the configurations; a batch forgets it when it builds its world anew. */
+int ugx_tile_select(ugx_case* c, int32_t variant);
 
 /* Device-to-device copy of `bytes` bytes timed over `reps` launches: the
  * stream-copy probe that confirms the HBM peak (no reference counterpart). */

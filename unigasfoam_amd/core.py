@@ -28,7 +28,8 @@ EXPORTS = [
     "ugx_wall_face_count", "ugx_wall_faces", "ugx_wall_samples_download", "ugx_wall_fields_compute",
     "ugx_cell_weights_download", "ugx_cell_weights_upload",
     "ugx_subcell_levels_download", "ugx_subcell_levels_upload", "ugx_time_get",
-    "ugx_phase_name", "ugx_timing_enable", "ugx_timing_get", "ugx_tile_config", "ugx_probe_copy",
+    "ugx_phase_name", "ugx_timing_enable", "ugx_timing_get", "ugx_tile_config", "ugx_tile_select",
+    "ugx_probe_copy",
     "ugx_batch_create", "ugx_batch_destroy", "ugx_case_footprint", "ugx_batch_admit", "ugx_batch_retire",
     "ugx_batch_step", "ugx_batch_sync", "ugx_batch_case", "ugx_batch_info",
 ]
@@ -92,6 +93,7 @@ def lib():
         L.ugx_probe_copy.argtypes = [C.c_int, C.c_int64, C.c_int, C.POINTER(C.c_double)]
         i32p = C.POINTER(C.c_int32)
         L.ugx_tile_config.argtypes = [vp, i32p, i32p, i32p, i32p, i32p]
+        L.ugx_tile_select.argtypes = [vp, C.c_int32]
         L.ugx_batch_create.argtypes = [C.POINTER(abi.BatchOptions), C.POINTER(vp)]
         L.ugx_batch_destroy.argtypes = [vp]
         L.ugx_case_footprint.argtypes = [C.POINTER(abi.MeshDesc), C.POINTER(abi.ModelDesc), C.c_int64, C.c_int,
@@ -444,6 +446,10 @@ class Case:
         check(self.L.ugx_tile_config(self.h, *[C.byref(x) for x in v]), self.L)
         return {"variant": v[0].value, "threads": v[1].value, "window": v[2].value, "lds_simulators": v[3].value,
                 "tuned": bool(v[4].value)}
+
+    def tile_select(self, variant):
+        """Run a cell-tile configuration (0 to 3) instead of the tuner's choice; -1: tune again."""
+        check(self.L.ugx_tile_select(self.h, int(variant)), self.L)
 
     def cell_volumes(self):
         out = np.zeros(self.nc)

@@ -3,6 +3,7 @@
 // returns a ugx_status and never lets a C++ exception cross the boundary.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstring>
 #include <new>
 #include <vector>
@@ -492,6 +493,20 @@ int ugx_tile_config(ugx_case* c, int32_t* variant, int32_t* threads, int32_t* wi
     if (window) *window = cfg[v][1];
     if (lds_simulators) *lds_simulators = cfg[v][2];
     if (tuned) *tuned = (!w->autotune || w->tune_step >= World::kTuneSteps) ? 1 : 0;
+    return UGX_OK;
+    UGX_GUARD_END
+}
+
+int ugx_tile_select(ugx_case* c, int32_t variant)
+{
+    UGX_GUARD_BEGIN
+    CHECK_CASE(c);
+    if (variant < -1 || variant >= kTileVariants) return set_err(UGX_ERR_ARG, "no cell-tile configuration %d", (int)variant);
+    World* w = c->world;
+    if (hipStreamSynchronize(w->stream) != hipSuccess) return set_err(UGX_ERR_DEVICE, "stream synchronize failed");
+    w->tile_variant = std::max(variant, 0);
+    w->tune_step = (variant < 0) ? 0 : World::kTuneSteps;
+    w->drop_graphs();
     return UGX_OK;
     UGX_GUARD_END
 }
