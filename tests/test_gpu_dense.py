@@ -14,13 +14,15 @@ from unigasfoam_amd.spec import Boundary, CaseSpec
 pytestmark = pytest.mark.gpu
 
 
-def phase_us(per_cell, crossings, phase, steps=3, n_cells=1000):
+def phase_us(per_cell, crossings, phase, steps=3, n_cells=1000, variant=-1):
     """Shortest time of a phase over `steps` steps of a channel whose simulators
     cross about `crossings` cells per step."""
     spec, fill = workloads.couette(n_cells=n_cells, per_cell=per_cell, dt=5.0e-9 * crossings, collision_model="none")
     g = Case(spec, precision="fp32", capacity=int(1.3 * n_cells * per_cell) + 70000)
     g.fill(**fill)
-    g.step(10)   # past the tuner's steps
+    if variant >= 0:
+        g.tile_select(variant)
+    g.step(2 if variant >= 0 else 10)   # past the tuner's steps
     best = float("inf")
     for _ in range(steps):
         g.timing(True)
@@ -76,3 +78,28 @@ def test_order_of_many_hits_on_many_faces(require_gpu):
                     collision_model="none", boundaries=[Boundary(p, abi.BND_SPECULAR) for p in pt])
     hits = same_wall_sums(spec, dict(number_density={"Ar": 2.0e19, "N2": 2.0e19}, T=300.0), 2, 1 << 23)
     assert 64 < hits < 256, hits
+
+
+@pytest.mark.parametrize("per_cell", [70, 140, 270, 1100, 6000])
+def test_merge_lists_match_oracle(require_gpu, per_cell):
+    """Merge lists of some 60 to 6000 slots, sorted 64 at a time: one stretch, an odd
+    and an even number of them."""
+    spec, fill = workloads.heat_bath(n_cells=2, per_cell=per_cell, side=2.0e-3, dt=1.0e-5)
+    g = Case(spec, precision="fp64", capacity=1 << 19)
+    o = OracleCase(spec, capacity=1 << 19)
+    for c in (g, o):
+        c.fill(**fill)
+    g.tile_select(3)
+    for c in (g, o):
+        c.step(3)
+    pg, po = g.particles(), o.particles()
+    for k in ("local", "velocity", "erot", "cell", "species"):
+        assert np.array_equal(pg[k], po[k]), k
+    g.close()
+    o.close()
+
+
+def test_merges_of_thousands_per_cell(require_gpu):
+    """Cells of 10,000 simulators of which most are merged by slot: the form
+    without tiles, whose merge lists have a wave, against tiles of 256 threads."""
+    assert phase_us(10000, 5, "cells", variant=3) < phase_us(10000, 5, "cells", variant=1)

@@ -1284,6 +1284,49 @@ __device__ inline void wall_terms(const double U[3], double e, const double n[3]
     t[UGX_W_ROTDOF] = (double)rotdof * inv;
 }
 
+// One pass of a merge sort by G lanes (lane j of them): ks[0..n) holds sorted
+// stretches of `run` distinct keys; put(q, d, key) takes the key of place q to its
+// place d among its stretch and the next one: its own number in its stretch plus
+// the number of smaller keys in the other.
+template <int G, class K, class Put>
+__device__ inline void merge_pass(const K* ks, uint32_t n, uint32_t run, uint32_t j, Put put)
+{
+    for (uint32_t q0 = 0; q0 < n; q0 += 4u * G) {
+        K mk[4];
+        uint32_t lo[4], hi[4], to[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const uint32_t q = min(q0 + j + G * (uint32_t)u, n - 1u);
+            const uint32_t first = q & ~(2u * run - 1u), second = min(first + run, n);
+            const bool in2 = (q & run) != 0u;
+            mk[u] = ks[q];
+            lo[u] = in2 ? first : second;
+            hi[u] = in2 ? second : min(second + run, n);
+            to[u] = first + (q - (in2 ? second : first)) - lo[u];
+        }
+        for (uint32_t s = run; s != 0u; s >>= 1) {
+            K k[4];
+            uint32_t mid[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                mid[u] = (lo[u] + hi[u]) >> 1;
+                k[u] = ks[min(mid[u], n - 1u)];
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const bool open = lo[u] < hi[u], less = k[u] < mk[u];
+                lo[u] = (open && less) ? mid[u] + 1u : lo[u];
+                hi[u] = (open && !less) ? mid[u] : hi[u];
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const uint32_t q = q0 + j + G * (uint32_t)u;
+            if (q < n) put(q, to[u] + lo[u], mk[u]);
+        }
+    }
+}
+
 // A group of G lanes per wall face: sorts the face's hits by key and adds
 // each species' terms in that order, then deltaT times the sums to the face's
 // time sums (at sample steps).  The order of the additions is fixed, so what
@@ -1349,51 +1392,17 @@ __global__ void __launch_bounds__(kBlock) k_wall_reduce(WorldView<R> w)
     }
     // a face of more hits: its sorted stretches merged pairwise, from the buckets to
     // the key list and back (the buckets hold what was in it; entries b.. are this
-    // face's to use), each hit's place being its own number in its stretch plus the
-    // number of smaller keys in the other one
+    // face's to use)
     bool alt = false;   // the order is in ev_key and ev.order, not in bkey and bidx
     for (uint32_t run = kKeys; run < n; run *= 2u) {
         __threadfence_block();
         wave_sync();
-        const unsigned long long* const ks = (alt ? w.ev_key : w.bkey) + b;
         unsigned long long* const kd = (alt ? w.bkey : w.ev_key) + b;
-        for (uint32_t q0 = 0; q0 < n; q0 += kKeys) {
-            unsigned long long mk[4];
-            uint32_t lo[4], hi[4], to[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const uint32_t q = min(q0 + j + G * (uint32_t)u, n - 1u);
-                const uint32_t first = q & ~(2u * run - 1u), second = min(first + run, n);
-                const bool in2 = (q & run) != 0u;
-                mk[u] = ks[q];
-                lo[u] = in2 ? first : second;
-                hi[u] = in2 ? second : min(second + run, n);
-                to[u] = first + (q - (in2 ? second : first)) - lo[u];
-            }
-            for (uint32_t s = run; s != 0u; s >>= 1) {
-                unsigned long long k[4];
-                uint32_t mid[4];
-#pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    mid[u] = (lo[u] + hi[u]) >> 1;
-                    k[u] = ks[min(mid[u], n - 1u)];
-                }
-#pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    const bool open = lo[u] < hi[u], less = k[u] < mk[u];
-                    lo[u] = (open && less) ? mid[u] + 1u : lo[u];
-                    hi[u] = (open && !less) ? mid[u] : hi[u];
-                }
-            }
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const uint32_t q = q0 + j + G * (uint32_t)u, d = to[u] + lo[u];
-                if (q >= n) continue;
-                kd[d] = mk[u];
-                if (alt) w.bidx[b + d] = w.ev[b + q].order;
-                else w.ev[b + d].order = w.bidx[b + q];
-            }
-        }
+        merge_pass<G>((alt ? w.ev_key : w.bkey) + b, n, run, j, [&](uint32_t q, uint32_t d, unsigned long long k) {
+            kd[d] = k;
+            if (alt) w.bidx[b + d] = w.ev[b + q].order;
+            else w.ev[b + d].order = w.bidx[b + q];
+        });
         alt = !alt;
     }
     if (!small) __threadfence_block();
@@ -2553,24 +2562,41 @@ __global__ void __launch_bounds__(kBlock) k_order(WorldView<R> w)
     wave_sync();
     if (oc != 0u && !big)
         for (uint32_t i = lo + j; i < e; i += 8u) w.perm[i] = w.scratch[i];
-    // the sorted merge list goes to the destination's cell ids, which the gather
-    // writes afterwards
-    uint32_t* sorted = w.b.cell;
+    // the merge list is sorted 64 slots at a time by rank, the stretches merged
+    // pairwise, from the slot list to the destination's cell ids (which the gather
+    // writes afterwards) and back (channel of 1e7 in 1000 cells, ten crossings per
+    // step: cells phase 9.3 ms; each slot ranked against the whole list 626, by tiles
+    // 36.  The lists of the cylinder are short: 141 us so, 155 like this)
     for (unsigned long long m = __ballot(big && j == 0u); m != 0ull; m &= m - 1ull) {
         const int src = __ffsll(m) - 1;
-        const uint32_t l = __shfl(lo, src), o = __shfl(eo, src), z = __shfl(e, src);
-        for (uint32_t i = o + lane; i < z; i += 64u) {
-            const uint32_t slot = w.perm[i];
-            uint32_t r = o;
-            for (uint32_t q = o; q < z; ++q) r += (w.perm[q] < slot) ? 1u : 0u;
-            sorted[r] = slot;
+        const uint32_t l = __shfl(lo, src), o = __shfl(eo, src), z = __shfl(e, src), n = z - o;
+        for (uint32_t q0 = o; q0 < z; q0 += 64u) {
+            const bool in = q0 + lane < z;
+            const uint32_t slot = in ? w.perm[q0 + lane] : 0xFFFFFFFFu;
+            uint32_t r = 0u;
+            auto below = [&](int q) { return ((uint32_t)__builtin_amdgcn_readlane((int)slot, q) < slot) ? 1u : 0u; };
+            if (z - q0 >= 64u) {
+#pragma unroll
+                for (int q = 0; q < 64; ++q) r += below(q);
+            } else {
+                for (int q = 0; q < (int)(z - q0); ++q) r += below(q);
+            }
+            if (in) w.perm[q0 + r] = slot;
+        }
+        const uint32_t* list = w.perm;
+        for (uint32_t run = 64u; run < n; run *= 2u) {
+            __threadfence_block();
+            wave_sync();
+            uint32_t* const to = (list == w.perm) ? w.b.cell : w.perm;
+            merge_pass<64>(list + o, n, run, lane, [&](uint32_t, uint32_t d, uint32_t slot) { to[o + d] = slot; });
+            list = to;
         }
         __threadfence_block();
         wave_sync();
         for (uint32_t i = l + lane; i < z; i += 64u) {
             const bool in = i < o;
-            const uint32_t slot = in ? w.perm[i] : sorted[i];
-            const uint32_t k = in ? lower_slot(sorted, o, z, slot) - o : lower_slot(w.perm, l, o, slot) - o;
+            const uint32_t slot = in ? w.perm[i] : list[i];
+            const uint32_t k = in ? lower_slot(list, o, z, slot) - o : lower_slot(w.perm, l, o, slot) - o;
             w.scratch[i + k] = slot;
         }
         __threadfence_block();
