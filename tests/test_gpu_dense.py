@@ -103,3 +103,14 @@ def test_merges_of_thousands_per_cell(require_gpu):
     """Cells of 10,000 simulators of which most are merged by slot: the form
     without tiles, whose merge lists have a wave, against tiles of 256 threads."""
     assert phase_us(10000, 5, "cells", variant=3) < phase_us(10000, 5, "cells", variant=1)
+
+
+def test_slow_configurations_are_timed_once(require_gpu):
+    """A dense world, where one configuration is more than twice as fast as another,
+    has its choice after fewer steps than two timings of all four would take."""
+    spec, fill = workloads.couette(n_cells=1000, per_cell=10000, collision_model="none")
+    g = Case(spec, precision="fp32", capacity=14000000)
+    g.fill(**fill)
+    g.step(7)
+    assert g.tile_config()["tuned"]
+    g.close()

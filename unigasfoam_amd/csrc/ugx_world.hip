@@ -1082,7 +1082,7 @@ int World::step(int n)
                 kn_due = 1;
                 kn_passes = std::max(kn_passes, c.smoothing_passes);
             }
-        // the tuner times each cell-tile configuration on two of the first
+        // the tuner times each cell-tile configuration on one or two of the first
         // kTuneSteps steps, with or without step timing
         // and, as the flow develops, it times the conservation kernel's two
         // occupancies on the collide phase of the last kConsVariants steps of
@@ -1138,9 +1138,13 @@ int World::step(int n)
             if (tile_tuning) {
                 HIP_TRY(hipEventElapsedTime(&ms, marks[6], marks[7]));
                 tune_ms[variant] = (tune_step < kTileVariants) ? (double)ms : std::min(tune_ms[variant], (double)ms);
-                if (++tune_step == kTuneSteps) {
-                    int best = 0;
-                    for (int v = 1; v < kTileVariants; ++v) if (tune_ms[v] < tune_ms[best]) best = v;
+                int best = 0;
+                for (int v = 1; v < kTileVariants; ++v) if (tune_ms[v] < tune_ms[best]) best = v;
+                ++tune_step;
+                while (tune_step >= kTileVariants && tune_step < kTuneSteps
+                       && tune_ms[tune_step % kTileVariants] > kTuneAgain * tune_ms[best])
+                    ++tune_step;
+                if (tune_step == kTuneSteps) {
                     tile_variant = best;
                     drop_graphs();
                 }
