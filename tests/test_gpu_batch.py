@@ -113,3 +113,33 @@ def test_admission_by_footprint(require_gpu):
     b.sync()
     assert b.info()["cases"] == 2
     b.close()
+
+
+def test_batch_tunes_again_when_its_size_changes(require_gpu):
+    """The cell-tile configuration is kept through rebuilds of about the size it was
+    chosen at, and chosen again past twice or below half of it."""
+    spec, fill = workloads.couette(n_cells=40, per_cell=20)
+    b = Batch(precision="fp32")
+    slots = []
+
+    def step_with(n_cases, steps):
+        while len(slots) < n_cases:
+            slots.append(b.admit(spec, fill, 2000))
+        b.step(steps)
+        b.sync()
+        return b.case(slots[0]).tile_config()["tuned"]
+
+    assert step_with(2, 8)
+    assert step_with(3, 1) and step_with(4, 1)     # up to twice the two cases
+    assert not step_with(5, 1)
+    assert step_with(5, 7)
+    assert step_with(10, 1)
+    assert not step_with(11, 1)
+    assert step_with(11, 7)
+    while len(slots) > 5:
+        b.retire(slots.pop())
+    assert step_with(6, 1)                          # six cases: half and more of eleven
+    for _ in range(2):
+        b.retire(slots.pop())
+    assert not step_with(5, 1)
+    b.close()

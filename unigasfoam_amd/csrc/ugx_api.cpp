@@ -506,6 +506,7 @@ int ugx_tile_select(ugx_case* c, int32_t variant)
     if (hipStreamSynchronize(w->stream) != hipSuccess) return set_err(UGX_ERR_DEVICE, "stream synchronize failed");
     w->tile_variant = std::max(variant, 0);
     w->tune_step = (variant < 0) ? 0 : World::kTuneSteps;
+    w->tuned_nc = w->tuned_cap = 0;
     w->drop_graphs();
     return UGX_OK;
     UGX_GUARD_END

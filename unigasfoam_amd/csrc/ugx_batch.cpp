@@ -86,12 +86,8 @@ static int rebuild(ugx_batch* b)
         nw->device = b->opt.device;
         if (int rc = nw->build(specs, b->opt.precision, b->opt.device, cap)) { delete nw; return rc; }
         nw->use_graphs = b->opt.use_graphs != 0;
-        if (b->world && b->world->tune_step >= World::kTuneSteps) {
-            // keep the tuned cell-tile configuration across rebuilds
-            nw->tile_variant = b->world->tile_variant;
-            nw->tune_step = b->world->tune_step;
-        }
         if (b->world) {
+            nw->take_tuning(*b->world);
             if (int rc = nw->adopt(*b->world, old_of_new)) { delete nw; return rc; }
         }
         bool filled = false;

@@ -1146,6 +1146,8 @@ int World::step(int n)
                     ++tune_step;
                 if (tune_step == kTuneSteps) {
                     tile_variant = best;
+                    tuned_nc = (uint64_t)nc;
+                    tuned_cap = cap;
                     drop_graphs();
                 }
             } else {
@@ -1532,6 +1534,16 @@ int World::pause(int ci)
 CellState World::cell_state()
 {
     return CellState{d_smax, d_cmodel, d_samp, d_uspq, d_usps, d_uspmax, d_knacc, d_kn, nc};
+}
+
+void World::take_tuning(const World& old)
+{
+    auto near = [](uint64_t a, uint64_t b) { return a <= 2u * b && b <= 2u * a; };
+    if (old.tune_step < kTuneSteps || !near((uint64_t)nc, old.tuned_nc) || !near(cap, old.tuned_cap)) return;
+    tile_variant = old.tile_variant;
+    tune_step = old.tune_step;
+    tuned_nc = old.tuned_nc;
+    tuned_cap = old.tuned_cap;
 }
 
 int World::adopt(World& old, const std::vector<int>& old_of_new)

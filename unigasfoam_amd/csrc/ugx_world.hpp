@@ -237,6 +237,10 @@ struct World {
     uint32_t move_grid = 0;       // resident blocks of the move kernel
     int tune_step = 0;
     double tune_ms[kTileVariants] = {};
+    uint64_t tuned_nc = 0, tuned_cap = 0;   // cells and slots when it was tuned
+    // takes the configuration of a world of a batch that this one replaces, unless
+    // it is more than twice or less than half the size that world was tuned at
+    void take_tuning(const World& old);
     // FP32 worlds with BGK-family cells and no macroInterpolation: the
     // conservation kernel's occupancy, re-timed every kConsRetune steps
     static constexpr uint64_t kConsRetune = 256;
