@@ -260,9 +260,13 @@ struct World {
     std::vector<CaseSpec> specs_host;
     std::vector<int64_t> samp_reset_steps;
     // Sampler downloads: kStageSlots parts of pinned host memory, each with an
-    // event, sized for the largest case and at most kStageBytes in all.
+    // event, sized for the largest case and at most kStageBytes in all.  A world's
+    // first download touches each page of it once, which at 16 MB cost more than
+    // the pinned path saved (17 MB: pageable 2.2 ms; first and later downloads with
+    // 16 MB 3.1 and 0.95, with 8 MB 2.0 and 0.9, with 4 MB 1.5 and 0.9 ms, but of
+    // 243 MB 9.0, 9.2 and 10.3 ms)
     static constexpr int kStageSlots = 4;
-    static constexpr size_t kStageBytes = size_t(16) << 20;
+    static constexpr size_t kStageBytes = size_t(8) << 20;
     static constexpr size_t kStageThreadBytes = size_t(1) << 20;   // larger downloads are copied by several threads
     std::mutex stage_mu;           // (cases of one world may be read by several threads)
     double* h_stage = nullptr;
