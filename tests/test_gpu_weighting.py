@@ -132,3 +132,24 @@ def test_weighted_fields_give_the_physical_density(require_gpu, precision):
     assert abs(rho.mean() / 1.0e20 - 1.0) < 0.2
     assert np.allclose(f["translational_T"].mean(), 300.0, rtol=0.02)
     g.close()
+
+
+def test_memory_of_the_clone_counts(require_gpu):
+    """Weighting holds a start cell and a clone count per slot (8 bytes) and an offset
+    per 1024 slots."""
+    import ctypes as C
+    hip = C.CDLL("libamdhip64.so")
+    cap = 1 << 26
+
+    def held(spec):
+        free, total = [C.c_size_t(), C.c_size_t()], C.c_size_t()
+        assert hip.hipMemGetInfo(C.byref(free[0]), C.byref(total)) == 0
+        g = Case(spec, precision="fp32", capacity=cap)
+        assert hip.hipMemGetInfo(C.byref(free[1]), C.byref(total)) == 0
+        g.close()
+        return free[0].value - free[1].value
+
+    plain = graded_box()
+    plain.cell_weighted = False
+    extra = held(graded_box()) - held(plain)
+    assert 8.0 * cap <= extra < 8.5 * cap, extra / cap

@@ -1028,12 +1028,7 @@ __global__ void __launch_bounds__(kBlock) k_wall(WorldView<R> w, uint32_t nwb)
 // Few simulators change weight, so the scan runs over a thousandth of the
 // slots (expansion of 1.2e7, 1e4 clones: weighting, scan and clones 211 us, like
 // this 122).
-constexpr uint32_t kCloneChunk = 4 * kBlock;
-
-__host__ __device__ inline uint32_t clone_chunks(uint32_t cap)
-{
-    return (uint32_t)(((uint64_t)cap + kCloneChunk - 1u) / kCloneChunk);
-}
+static_assert(kCloneChunk == 4 * kBlock, "four slots per thread");
 
 // Exclusive scan of v over the block's threads; total is the block's sum.
 __device__ inline uint32_t block_excl_scan(uint32_t v, uint32_t& total)
@@ -2499,6 +2494,16 @@ __global__ void __launch_bounds__(Block) __attribute__((amdgpu_waves_per_eu((NS 
     }
 }
 
+// First of the entries [lo, hi) of p (ascending) that is not below v.
+__device__ inline uint32_t lower_slot(const uint32_t* p, uint32_t lo, uint32_t hi, uint32_t v)
+{
+    while (lo < hi) {
+        const uint32_t mid = (lo + hi) >> 1;
+        if (p[mid] < v) lo = mid + 1u; else hi = mid;
+    }
+    return lo;
+}
+
 // The same three steps without tiles, for dense cells: there a tile holds one
 // cell, more than LDS takes, so that k_tile's gather waits for its slot list
 // and its sums run on eight lanes of its block.  Here
@@ -2514,15 +2519,6 @@ __global__ void __launch_bounds__(Block) __attribute__((amdgpu_waves_per_eu((NS 
 // + 356 without; expansion of 1.2e7, 50 per cell: 373 and 348; heat bath of
 // 3.6e5, 30 per cell and most of them to be merged: 25 and 52).  The tuner
 // takes this form where it is faster.
-// First of the entries [lo, hi) of p (ascending) that is not below v.
-__device__ inline uint32_t lower_slot(const uint32_t* p, uint32_t lo, uint32_t hi, uint32_t v)
-{
-    while (lo < hi) {
-        const uint32_t mid = (lo + hi) >> 1;
-        if (p[mid] < v) lo = mid + 1u; else hi = mid;
-    }
-    return lo;
-}
 
 // Largest reordering that the eight lanes of a cell do by themselves; a larger
 // one takes the wave.  The cells of a wave lie a grid apart, so that a row of
@@ -3127,12 +3123,9 @@ __global__ void __launch_bounds__(kBlock) k_collide(WorldView<R> w, uint32_t spr
         const CaseDev& cs = w.cases[ccase];
         BgkP P;
         bgk_params<R>(w, cs, c, nC, S, P, nrel);
+        P.nrel = nrel;
         w.bgkp[c] = P;
         w.raise[c] = 0ull;
-    }
-    if (bgk) {
-        w.bgkp[c].sel_base = b;
-        w.bgkp[c].nrel = nrel;
     }
     __shared__ uint16_t s_perm[kSelLds * kBlock];
     if (nrel) bgk_select<R>(w, w.cases[ccase], c, b, nC, nrel, b, A, &s_perm[threadIdx.x]);
@@ -3450,7 +3443,7 @@ __device__ __attribute__((always_inline)) inline void bgk_conserve_body(const Wo
             const BgkP& P = w.bgkp[c];
             perform = P.perform != 0;
             usp = P.model == UGX_BGK_USP;
-            sb = P.sel_base;
+            sb = cb;   // (a cell's selections are listed from its first slot on)
             nrel = P.nrel;
             if (perform) {
                 b = cb;

@@ -43,7 +43,6 @@ struct BgkP {
     double sm[9];      // ES-BGK S matrix (row major) or USP stress (xx xy xz yy yz zz)
     int32_t perform;
     int32_t model;
-    uint32_t sel_base;  // first entry of the cell's selections in the selection list
     uint32_t nrel;      // number of selections
 };
 
@@ -53,6 +52,13 @@ inline size_t scan_bsum_words(uint64_t n)
 {
     const size_t nb = (size_t)((n + 1023) / 1024);
     return nb + 1 + (nb + 1023) / 1024 + 2;
+}
+
+// Slots whose clones the cell weighting counts together.
+constexpr uint32_t kCloneChunk = 1024;
+__host__ __device__ inline uint32_t clone_chunks(uint32_t cap)
+{
+    return (uint32_t)(((uint64_t)cap + kCloneChunk - 1u) / kCloneChunk);
 }
 
 // Per-case cumulative counters (uint64).
@@ -161,8 +167,8 @@ struct WorldView {
     int32_t has_weighting;
     uint32_t* cstart;         // [cap]
     uint32_t* wclone;         // [cap + 1] clone count of a slot
-    uint32_t* wcoff;          // [cap + 1] per chunk of slots its clones, then the offset of the first
-    uint32_t* wbsum;          // scan scratch for cap entries
+    uint32_t* wcoff;          // [clone_chunks(cap) + 1] per chunk of slots its clones, then the offset of the first
+    uint32_t* wbsum;          // scan scratch for those
     // NTC subcells (noTimeCounter.C:97-161): with any cell split, per cell
     // its packed levels (x | y << 8 | z << 16) and the offset of its subcell
     // table (2 nsub + 1 words: subcell starts, then cursors), per slot of

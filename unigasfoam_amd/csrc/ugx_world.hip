@@ -450,8 +450,8 @@ int World::alloc_particles(uint32_t newcap)
         dfree(d_wbsum);
         if (int rc = dalloc(d_cstart, newcap)) return rc;
         if (int rc = dalloc(d_wclone, (size_t)newcap + 1)) return rc;
-        if (int rc = dalloc(d_wcoff, (size_t)newcap + 1)) return rc;
-        if (int rc = dalloc(d_wbsum, scan_bsum_words((uint64_t)newcap + 1))) return rc;
+        if (int rc = dalloc(d_wcoff, (size_t)clone_chunks(newcap) + 1)) return rc;
+        if (int rc = dalloc(d_wbsum, scan_bsum_words((uint64_t)clone_chunks(newcap) + 1))) return rc;
     }
     if (has_subcells) {
         dfree(d_scid);
