@@ -477,9 +477,11 @@ int ugx_batch_info(ugx_batch* b, int64_t* n_cases, int64_t* bytes_used, int64_t*
 /* Per-phase timing of ugx_step with HIP events on the case's stream (no
  * counterpart in the reference, whose only timing is the ExecutionTime /
  * ClockTime log line of uniGasFoam.C:97-101).  Phases, in launch order:
- * begin, inflow, move, wall (diffuse-wall continuation), scan, scatter,
- * cells (slot order + gather + per-cell sums + sampler), collide (NTC and
- * the BGK family), end. */
+ * begin (with the inflow counts of up to 4096 face-species), inflow (the
+ * counts of more), move, wall (diffuse-wall continuation beside the new
+ * simulators, wall sums, cell weighting and clones), scan, scatter, cells
+ * (slot order + gather + per-cell sums + sampler), collide (NTC and the BGK
+ * family, hybrid decomposition), end. */
 #define UGX_N_PHASES 9
 const char* ugx_phase_name(int i);
 int ugx_timing_enable(ugx_case* c, int on);       /* also resets the totals */

@@ -1450,9 +1450,13 @@ __global__ void __launch_bounds__(kBlock) k_wall_reduce(WorldView<R> w)
     if (j < (uint32_t)kWRows && ls >= 0) sums[(size_t)ls * kWRows + j] += dt * a;
 }
 
-// Up to this many wall faces a wave each: the waves are then resident at once
-// (256 CUs x 32).  More faces (a 3-D mesh, few hits each) take 16 lanes each:
-// 45,000 faces with one hit each take 21 us (23 us with a thread per face).
+// Up to this many wall faces a wave each, more (a 3-D mesh) 16 lanes each.  The 38 KB
+// of LDS of a block leave room for 4096 waves at once, so faces of few hits are
+// better off with 16 lanes from about there on, faces of many hits with 64 up to
+// twice that (wall phase, 64 / 16 lanes, us): 7.5 hits per face: 4056 faces 25.0 /
+// 26.6, 5400 30.6 / 27.6, 8214 36.6 / 30.6, 21,600 (5 hits) 56 / 36; 37 hits: 5400
+// 49 / 53, 8214 60 / 58, 11,616 76 / 67; 75 hits: 5400 69 / 84; 100 hits: 4056
+// 66 / 107.
 constexpr int32_t kWallWaveFaces = 8192;
 
 // ------------------------------------------------------------ occupancy
@@ -1476,7 +1480,12 @@ constexpr uint32_t kMaxTileCells = 512u / kCellW + 2u;   // cells of the largest
 constexpr int kCountTiles = 4;                           // tiles per block of k_count_tiles
 // Largest grid of the occupancy count (blocks stride over the step's tile groups).
 constexpr uint64_t kCountGrid = 8192;
-// Tile tables up to this length get a block per tile.
+// Tile tables up to this length (its bound for the capacity) get a block per tile.
+// Scan phase with one and with four tiles per block, us: channel of 1e5 18.5 and 31,
+// bath of 3.6e5 26 and 36; just above the line some worlds still prefer one (FP64
+// cylinder of 7.7e5 28 and 38), others, with many simulators that crossed several
+// cells, do not (baths of 1e6, 200 and 400 per cell: 62 and 51, 93 and 69); large ones
+// do not (expansion of 1.2e7 198 and 141, mixed nozzle of 4.2e7 667 and 456).
 constexpr uint64_t kCountSmall = 8192;
 
 // Class-7 counting of the slots [begin, n + n_ins) as block `block` of
@@ -2829,7 +2838,9 @@ __device__ inline void ntc_cell(const WorldView<R>& w, const CaseDev& cs, uint32
         // sigma_T c_r = C cR2^e against u smax0: nearly every candidate is decided by
         // the hardware's single-precision log2 and exp2.  Their result q is within
         // 2e-5 of sigma_T c_r / smax0 (one unit in the last place of |log2| <= 100,
-        // twice, times |e| <= 1, and four roundings); where u or the running maximum
+        // twice, times |e| <= 1, and four roundings; C / smax0 would have to be below
+        // 1e-38 for its own rounding to matter, and q then clears 1e-30 only at
+        // relative speeds above 1e11 m/s); where u or the running maximum
         // is within 1e-4 of it, or the numbers leave the guarded range, the double
         // value decides and raises the maximum.  With it, and the candidate's and
         // the collision's numbers drawn together, k_collide went from 111 to 89 us
@@ -4245,7 +4256,11 @@ static inline bool count_shared(uint32_t nc, uint64_t cap) { return cap >= kCoun
 // and more per cell) over as many as are resident (channel of 500 cells of 200:
 // 33 us, 22; FP64 cylinder of 5141 of 150: 73, 50; cylinder of 8e4 of 625: 477,
 // 402).  Cells of 40 gain nothing past one wave per SIMD and lose memory
-// coalescing (DSMC nozzle of 5.9e4 cells: 92 us, spread over 1832 waves 102).
+// coalescing (DSMC nozzle of 5.9e4 cells: 92 us, spread over 1832 waves 102).  Near
+// the line the two limits differ by less than a tenth (collisions of argon
+// channels, kCollideWaves and kCollideWavesDense, us: 2000 cells of 100 14.5 and
+// 14.5, of 300 23.2 and 21.5, of 600 35.9 and 30.7; 20,000 cells of 100 17.9 and
+// 19.4, of 300 30.3 and 31.6; 1e5 cells of 150 51.9 and 51.8).
 constexpr uint64_t kCollideWaves = 1536, kCollideWavesDense = 3072, kDenseCell = 128;
 
 static inline uint32_t collide_spread(uint32_t nc, uint64_t cap)
