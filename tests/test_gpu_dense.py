@@ -106,8 +106,17 @@ def test_merges_of_thousands_per_cell(require_gpu):
 
 
 def test_slow_configurations_are_timed_once(require_gpu):
-    """A dense world, where one configuration is more than twice as fast as another,
-    has its choice after fewer steps than two timings of all four would take."""
+    """A dense world, where some configurations take milliseconds and more than twice
+    the fastest, has its choice after fewer steps than two timings of all four would
+    take; a small one, where a kernel's first launch may look as slow, times all twice."""
+    spec, fill = workloads.couette(n_cells=20, per_cell=20, collision_model="none")
+    g = Case(spec, precision="fp32", capacity=1000)
+    g.fill(**fill)
+    g.step(7)
+    assert not g.tile_config()["tuned"]
+    g.step(1)
+    assert g.tile_config()["tuned"]
+    g.close()
     spec, fill = workloads.couette(n_cells=1000, per_cell=10000, collision_model="none")
     g = Case(spec, precision="fp32", capacity=14000000)
     g.fill(**fill)

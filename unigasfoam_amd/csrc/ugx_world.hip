@@ -1142,7 +1142,7 @@ int World::step(int n)
                 for (int v = 1; v < kTileVariants; ++v) if (tune_ms[v] < tune_ms[best]) best = v;
                 ++tune_step;
                 while (tune_step >= kTileVariants && tune_step < kTuneSteps
-                       && tune_ms[tune_step % kTileVariants] > kTuneAgain * tune_ms[best])
+                       && tune_ms[tune_step % kTileVariants] > std::max(kTuneWorth, kTuneAgain * tune_ms[best]))
                     ++tune_step;
                 if (tune_step == kTuneSteps) {
                     tile_variant = best;

@@ -224,14 +224,14 @@ struct World {
     bool use_graphs = false;
     // autotuner: each of the first kTuneSteps steps at most times one cell-tile
     // configuration on the live case (results do not depend on it).  The first
-    // launch of a kernel is slow and irregular (channel of 1e5, FP32: timed once, a
-    // configuration of 36 us was taken where another ran in 21), so those that
-    // took up to kTuneAgain times the fastest are timed again, the faster time
-    // counting; the others, slow steps in a large world, are not (channel of 1e7 in
-    // 1000 cells, ten crossings per step, 9 ms a step: its first eight steps 500 ms
-    // with all four timed twice, 290 like this)
+    // launch of a kernel in a process takes 0.1 to 0.25 ms longer (channels of 1e4
+    // to 1e5: 144 us, then 15), so every configuration is timed twice, the faster time
+    // counting.  Those that took more than kTuneWorth ms and kTuneAgain times the
+    // fastest are not timed again: that cannot be a first launch's, and their steps
+    // are slow ones (channel of 1e7 in 1000 cells, ten crossings per step, 9 ms a
+    // step: its first eight steps 500 ms with all four timed twice, 290 like this)
     static constexpr int kTuneSteps = 2 * kTileVariants;
-    static constexpr double kTuneAgain = 2.0;
+    static constexpr double kTuneAgain = 2.0, kTuneWorth = 1.0;
     bool autotune = true;
     int tile_variant = 0;
     uint32_t move_grid = 0;       // resident blocks of the move kernel
