@@ -38,13 +38,16 @@ COLLISION_DESC = {"hybrid": "hybrid USP/DSMC (NTC+VHS)", "dsmc": "DSMC (NTC+VHS)
 # --pmc FETCH_SIZE and WRITE_SIZE runs of this bench line (FETCH_SIZE scaled by
 # 2 and WRITE_SIZE by 1, the factors a 2 GiB copy kernel reads; averages of the
 # last 20 launches; the profile summary named beside each holds the tables).
+# The cells phase by cell-tile configuration; one that was not profiled has none.
 PMC_TRAFFIC = {
     "expansion": {"profile": "profiles/nozzle_expansion_1e8_fp32.md",
-                  "collide": (0.71 + 0.95 + 2.41 + 2.69) * 1e9,      # k_collide + k_bgk_conserve5
-                  "cells": (9.59 + 4.56) * 1e9, "move": (4.24 + 2.07) * 1e9},
+                  "collide": (0.71 + 0.95 + 2.75 + 3.24) * 1e9,      # k_collide + k_bgk_conserve5
+                  "cells": {0: (9.93 + 4.67) * 1e9, 1: (10.04 + 4.59) * 1e9, 3: (13.10 + 4.61) * 1e9},
+                  "move": (4.27 + 2.06) * 1e9},
     "nozzle": {"profile": "profiles/nozzle_1e8_fp32.md",
-               "collide": (0.78 + 0.63 + 2.00 + 1.56) * 1e9,      # k_collide + k_bgk_conserve5
-               "cells": (12.01 + 4.71) * 1e9, "move": (4.31 + 1.61) * 1e9},
+               "collide": (0.78 + 0.67 + 2.16 + 1.43) * 1e9,      # k_collide + k_bgk_conserve<float, false>
+               "cells": {0: (12.01 + 4.71) * 1e9, 1: (11.67 + 4.60) * 1e9, 3: (15.06 + 4.62) * 1e9},
+               "move": (4.35 + 1.61) * 1e9},
 }
 
 
@@ -336,7 +339,10 @@ def main():
     achieved = dom_bytes / dom_s / 1e9
     step_b = roofline.step_bytes(R, n_avg, nc, cand, coll, n_bgk, **kw)
     pm = PMC_TRAFFIC.get(args.workload, {}) if (args.scale == 1.0 and args.precision == "fp32") else {}
-    traffic = int(pm[dom]) if dom in pm else None
+    traffic = pm.get(dom)
+    if isinstance(traffic, dict):
+        traffic = traffic.get(case.tile_config()["variant"])
+    traffic = int(traffic) if traffic else None
     traffic_src = (pm["profile"] + " (rocprofv3 --pmc FETCH_SIZE x2 + WRITE_SIZE)") if traffic else None
     step_gbs = step_b / (elapsed / args.steps) / 1e9
     out = {
