@@ -493,7 +493,8 @@ int ugx_timing_get(ugx_case* c, double* ms_total, int n_phases, int64_t* steps);
  * configurations (the last works without tiles: no LDS simulators) on one of
  * the case's first four steps and on one of the next four (except those that
  * took over 1 ms and over twice the fastest), with or without
- * ugx_timing_enable, and keeps the fastest; results never depend on it. */
+ * ugx_timing_enable, and keeps the one with the least time in the cells phase
+ * and in the next step's count; results never depend on it. */
 int ugx_tile_config(ugx_case* c, int32_t* variant, int32_t* threads, int32_t* window, int32_t* lds_simulators,
                     int32_t* tuned);
 /* Runs configuration `variant` (0 to 3) from the next step on instead of the

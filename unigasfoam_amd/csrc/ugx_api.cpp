@@ -5,6 +5,7 @@
 
 #include <algorithm>
 #include <cstring>
+#include <iterator>
 #include <new>
 #include <vector>
 
@@ -507,6 +508,8 @@ int ugx_tile_select(ugx_case* c, int32_t variant)
     w->tile_variant = std::max(variant, 0);
     w->tune_step = (variant < 0) ? 0 : World::kTuneSteps;
     w->tuned_nc = w->tuned_cap = 0;
+    std::fill(std::begin(w->tune_count_ms), std::end(w->tune_count_ms), 0.0);
+    w->tune_last = w->tile_variant;
     w->drop_graphs();
     return UGX_OK;
     UGX_GUARD_END

@@ -1138,8 +1138,14 @@ int World::step(int n)
             if (tile_tuning) {
                 HIP_TRY(hipEventElapsedTime(&ms, marks[6], marks[7]));
                 tune_ms[variant] = (tune_step < kTileVariants) ? (double)ms : std::min(tune_ms[variant], (double)ms);
+                // the count of this step ran over the table of the last one's windows
+                HIP_TRY(hipEventElapsedTime(&ms, marks[4], marks[5]));
+                double& count_ms = tune_count_ms[tile_table(tune_last)];
+                count_ms = (count_ms == 0.0) ? (double)ms : std::min(count_ms, (double)ms);
+                tune_last = variant;
+                auto score = [&](int v) { return tune_ms[v] + tune_count_ms[tile_table(v)]; };
                 int best = 0;
-                for (int v = 1; v < kTileVariants; ++v) if (tune_ms[v] < tune_ms[best]) best = v;
+                for (int v = 1; v < kTileVariants; ++v) if (score(v) < score(best)) best = v;
                 ++tune_step;
                 while (tune_step >= kTileVariants && tune_step < kTuneSteps
                        && tune_ms[tune_step % kTileVariants] > std::max(kTuneWorth, kTuneAgain * tune_ms[best]))

@@ -237,6 +237,13 @@ struct World {
     uint32_t move_grid = 0;       // resident blocks of the move kernel
     int tune_step = 0;
     double tune_ms[kTileVariants] = {};
+    // Occupancy count over the tile table of each window, counted into a
+    // configuration's time (mixed nozzle of 1e8: 256-key windows are 0.02 ms faster
+    // in the cells phase and 0.07 ms slower in the next step's count), and the
+    // configuration whose table the next count runs over
+    double tune_count_ms[kTileVariants] = {};
+    int tune_last = 0;
+    static int tile_table(int variant) { return variant == kTilesNone ? 0 : variant; }
     uint64_t tuned_nc = 0, tuned_cap = 0;   // cells and slots when it was tuned
     // takes the configuration of a world of a batch that this one replaces, unless
     // it is more than twice or less than half the size that world was tuned at
