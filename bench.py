@@ -42,12 +42,12 @@ COLLISION_DESC = {"hybrid": "hybrid USP/DSMC (NTC+VHS)", "dsmc": "DSMC (NTC+VHS)
 PMC_TRAFFIC = {
     "expansion": {"profile": "profiles/nozzle_expansion_1e8_fp32.md",
                   "collide": (0.71 + 0.95 + 2.75 + 3.24) * 1e9,      # k_collide + k_bgk_conserve5
-                  "cells": {0: (9.93 + 4.67) * 1e9, 1: (10.04 + 4.59) * 1e9, 3: (13.10 + 4.61) * 1e9},
-                  "move": (4.27 + 2.06) * 1e9},
+                  "cells": {0: (9.93 + 4.67) * 1e9, 1: (9.59 + 4.56) * 1e9, 3: (13.10 + 4.61) * 1e9},
+                  "move": (4.28 + 2.06) * 1e9},
     "nozzle": {"profile": "profiles/nozzle_1e8_fp32.md",
                "collide": (0.78 + 0.67 + 2.16 + 1.43) * 1e9,      # k_collide + k_bgk_conserve<float, false>
-               "cells": {0: (12.01 + 4.71) * 1e9, 1: (11.67 + 4.60) * 1e9, 3: (15.06 + 4.62) * 1e9},
-               "move": (4.35 + 1.61) * 1e9},
+               "cells": {0: (12.01 + 4.71) * 1e9, 1: (11.20 + 4.58) * 1e9, 3: (15.07 + 4.62) * 1e9},
+               "move": (4.36 + 1.61) * 1e9},
 }
 
 
