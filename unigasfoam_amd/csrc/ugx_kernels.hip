@@ -1536,7 +1536,7 @@ __global__ void k_count(WorldView<R> w)
 constexpr uint32_t kCountWindow = 512;
 
 // Shared: with an atomic per distinct key (an instance of its own: as a branch it
-// cost the other form 1 to 6%, expansion of 1e8 994 us, 1050).
+// cost both forms 1%; scan phase of the mixed nozzle of 4.2e7 450 us, 456).
 template <class R, int Block, int TPB, bool Shared>
 __global__ void __launch_bounds__(Block) __attribute__((amdgpu_waves_per_eu(7))) k_count_tiles(WorldView<R> w, uint32_t ntb, uint32_t tpb)
 {
