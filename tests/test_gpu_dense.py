@@ -40,7 +40,6 @@ def test_count_of_cells_crossed(require_gpu):
     assert phase_us(10000, 2, "scan", variant=1) < 1.7 * phase_us(10000, 0.02, "scan", variant=1)
 
 
-
 def test_sums_of_many_hits_per_face(require_gpu):
     """Ten times the hits on the two faces of a channel (570 and 5700 each)."""
     assert phase_us(1000, 10, "wall") < 20.0 * phase_us(1000, 1, "wall")
